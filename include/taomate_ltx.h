@@ -251,6 +251,23 @@ int ltx_flash_attn_fwd(const void* q, int64_t B, int64_t Lq, int64_t H, int64_t 
                        int64_t workspace_bytes, void* stream);
 
 /*
+ * ltx_flash_attn_fwd over plain cache tensors: token-major bf16 K and V whose
+ * segments are separate tensors with their own batch strides, as the
+ * reference holds them before torch.cat (ltx_causal/transformer/
+ * kv_cache.py:1487-1491), attended where they lie instead of concatenated.
+ *   Segment i: K and V at k_ptrs[i], v_ptrs[i], element (b, t, h, d) at
+ *   b*seg_bs[i] + t*kv_ls + h*kv_hs + d (seg_bs: a host array, read during the
+ *   call; token and head strides shared by all).  Other arguments as
+ *   ltx_flash_attn_fwd.
+ */
+int ltx_flash_attn_fwd_plain(const void* q, int64_t B, int64_t Lq, int64_t H, int64_t D, int64_t q_bs,
+                             int64_t q_ls, int64_t q_hs, int64_t n_segments, const void* const* k_ptrs,
+                             const void* const* v_ptrs, const int64_t* seg_lens, const int64_t* seg_bs,
+                             int64_t kv_ls, int64_t kv_hs, void* out, int64_t o_bs, int64_t o_ls,
+                             int64_t o_hs, float* lse, float scale, void* workspace,
+                             int64_t workspace_bytes, void* stream);
+
+/*
  * ltx_flash_attn_fwd without a workspace argument, for callers that cannot
  * allocate device memory (code under HIP graph capture, tight serving loops,
  * harnesses that forbid hipMalloc).  No counterpart in the reference.

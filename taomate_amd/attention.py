@@ -343,34 +343,23 @@ def standard_attention_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
     return out
 
 
-def _dense_segments(segs: List[KVSegment], new_k: torch.Tensor, new_v: torch.Tensor,
-                    n_queries: int) -> List[KVSegment]:
+def _dense_segments(segs: List[KVSegment], new_k: torch.Tensor, new_v: torch.Tensor) -> List[KVSegment]:
     """Segments for a plain-tensor cache (the reference's torch.cat caches) plus
-    the new chunk.  K is concatenated as the reference does (kv_cache.py:
-    1487-1491) when the cache tensor's strides differ from the chunk's.  V goes
-    into one key-major store instead of a token-major concatenation, the same
-    bytes moved, so the attention runs on the pipelined kernel rather than the
-    staged one (measured at 1152 queries over 3456 cached + 1152 new keys,
-    B = 2, 32 x 128: 236 us staged, 180 us pipelined)."""
+    the new chunk: the cache tensors and the chunk's are attended where they
+    lie, on the token-major instance of the pipelined kernel, when they share
+    token and head strides; else they are concatenated as the reference does
+    (kv_cache.py:1487-1491).  (Concatenating K and copying V into a key-major
+    store took 105 of the layer's 530 us at 1152 queries over 3456 cached +
+    1152 new keys, B = 2, 32 x 128.)"""
     if not segs:
         return [KVSegment(new_k, new_v)]
     old = segs[0]
-    B, Lc, H, D = old.v.shape
-    Ln = new_v.shape[1]
-    same = old.k.stride() == new_k.stride()
-    if D not in (64, 128) or n_queries < 256 or Lc + Ln < 64 or Lc % 8:
-        if same and old.v.stride() == new_v.stride():
-            return segs + [KVSegment(new_k, new_v)]
-        return [KVSegment(torch.cat([old.k, new_k], dim=1), torch.cat([old.v, new_v], dim=1))]
-    store = torch.empty(B, H, D, -(-(Lc + Ln) // 8) * 8, dtype=new_v.dtype, device=new_v.device)
-    if store.shape[-1] > Lc + Ln:
-        store[..., Lc + Ln:].zero_()
-    vkm = store.permute(0, 3, 1, 2)
-    kernels.kv_append(old.v, vkm[:, :Lc])
-    kernels.kv_append(new_v, vkm[:, Lc:Lc + Ln])
-    if same:
-        return [KVSegment(old.k, vkm[:, :Lc]), KVSegment(new_k, vkm[:, Lc:Lc + Ln])]
-    return [KVSegment(torch.cat([old.k, new_k], dim=1), vkm[:, :Lc + Ln])]
+    inner = new_k.stride()[1:]
+    if all(t.stride()[1:] == inner and t.data_ptr() % 16 == 0 and t.stride(0) % 8 == 0
+           for t in (old.k, old.v, new_k, new_v)) and inner[2] == 1 and inner[0] % 8 == 0 and inner[1] % 8 == 0 \
+            and old.k.stride(0) == old.v.stride(0) and new_k.stride(0) == new_v.stride(0):
+        return segs + [KVSegment(new_k, new_v)]
+    return [KVSegment(torch.cat([old.k, new_k], dim=1), torch.cat([old.v, new_v], dim=1))]
 
 
 def _cached_segments(cached_k, cached_v) -> Tuple[List[KVSegment], int]:
@@ -462,9 +451,10 @@ def attention_with_cache(
         if not new_v.is_contiguous() or (segs and segs[0].k.stride() != new_k.stride()):
             new_v = new_v.contiguous()
             new_k = new_k.contiguous()
-        segs = _dense_segments(segs, new_k, new_v, L)
+        segs = _dense_segments(segs, new_k, new_v)
     if logit_log_scale is not None:
         q = q * logit_log_scale
     out = torch.empty(B, L, H, D, dtype=q.dtype, device=q.device)
-    kernels.flash_attn(q.view(B, L, H, D), segs, out, frame_tokens=frame)
+    kernels.flash_attn(q.view(B, L, H, D), segs, out, frame_tokens=frame,
+                       segment_batch_strides=arena is None and len(segs) > 1)
     return _finish(attn, out, x), new_k, new_v

@@ -52,7 +52,8 @@ struct FlashParams {
   int64_t q_bs, q_ls, q_hs;
   int64_t o_bs, o_ls, o_hs;
   int o_al16;                        // o and its strides are 16-byte aligned (staged output stores)
-  int64_t kv_bs, kv_ls, kv_hs;      // K (and token-major V) strides
+  int64_t kv_ls, kv_hs;              // K (and token-major V) token and head strides
+  int64_t seg_bs[LTX_MAX_SEGMENTS];  // and each segment's batch stride, in bytes
   int64_t v_bs, v_hs, v_ds;          // key-major V: element (b, t, h, d) at b*v_bs + h*v_hs + d*v_ds + t
   int64_t sc_bs, sc_hs;
   int64_t mask_bs;
@@ -120,6 +121,13 @@ __device__ __forceinline__ int sig(int r) { return (r & ~12) | ((r & 4) << 1) | 
 // a lane's scores of two adjacent 16-key blocks are 8 consecutive keys.
 template <int NC>
 __host__ __device__ constexpr int row_swizzle(int r) { return NC == 16 ? (r & 15) : ((r >> 1) & 7); }
+// chunk pairs of a token-major V tile's key rows: the 8 keys that half a
+// transposing fragment read touches (two blocks of 4, 8 keys apart, one 32-byte
+// chunk pair each) fall on 8 different 32-byte bank groups
+template <int NC>
+__host__ __device__ constexpr int key_swizzle(int r) {
+  return NC == 16 ? 2 * ((r & 3) | ((r >> 1) & 4)) : 2 * (((r >> 1) & 1) | ((r >> 2) & 2));
+}
 __host__ __device__ constexpr int key_of_row(int r) { return (r & 35) | ((r & 12) << 1) | ((r & 16) >> 2); }
 
 // Blocks are dispatched round-robin over the 8 XCDs (block id % 8).  Give each
@@ -511,8 +519,10 @@ __global__ void __launch_bounds__(256) flash_combine_kernel(const FlashParams p)
   if (p.lse != nullptr && cg == 0) p.lse[((int64_t)b * p.H + h) * p.Lq + q] = (mmax + __log2f(lsum)) / kLog2e;
 }
 
-template <int D, bool FP8, bool MASK>
-__global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const FlashParams p) {
+// Register-staged kernel for calls with an additive key mask (bf16, token-major
+// V): the mask joins the logits, so the softmax takes every tile's maximum.
+template <int D>
+__global__ void __launch_bounds__(256, 2) flash_fwd_masked_kernel(const FlashParams p) {
   constexpr int BM = kBM, BN = kBN;
   constexpr int KS = D + 8;                // K tile LDS row stride (elements)
   constexpr int VS = BN + 8;               // V^T tile LDS row stride
@@ -524,11 +534,11 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const FlashParams p) 
   constexpr int NVP = (BN / 4) * (D / 8);  // (4-key group, 8-d chunk) pairs
   constexpr int DB = D / 32;
   constexpr int QS = D / 16;
-  using Chunk = KVChunk<FP8>;
+  using Chunk = KVChunk<false>;
   using raw_t = typename Chunk::raw_t;
 
   __shared__ __attribute__((aligned(16))) uint16_t smem[2 * (KBUF + VBUF)];
-  __shared__ float mask_s[MASK ? 2 : 1][MASK ? BN : 1];
+  __shared__ float mask_s[2][BN];
 
   const WorkItem wi = work_item(p, blockIdx.x, p.tile_start[p.n_seg]);
   const int qt = wi.qtile % p.n_qtiles;
@@ -551,14 +561,14 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const FlashParams p) 
     }
   }
 
-  const int64_t kv_off = b * p.kv_bs + h * p.kv_hs;
+  const int64_t kv_off = h * p.kv_hs;
   // rows this thread moves in every tile, as loop-invariant byte offsets from
   // the tile's first row (buffer loads return 0 past the tile's valid rows)
   const int kc = tid % NKC;
   const int kr0 = tid / NKC;
   const int vkg = tid % 16, vdc = tid / 16;
   const bool vthread = tid < NVP;
-  constexpr int ESZ = FP8 ? 1 : 2;
+  constexpr int ESZ = 2;
   const int row_bytes = (int)(p.kv_ls * ESZ);
   int koff[K_LOADS], voff[4];
 #pragma unroll
@@ -573,7 +583,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const FlashParams p) 
   TileIter ld;
   ld.seek(p, wi.j0);
   auto load_tile = [&]() {
-    const int64_t base = (kv_off + ld.row0 * p.kv_ls) * ESZ;
+    const int64_t base = b * p.seg_bs[ld.s] + (kv_off + ld.row0 * p.kv_ls) * ESZ;
     const int nbytes = ld.nvalid() * row_bytes;
     const auto kr = __builtin_amdgcn_make_buffer_rsrc(
         (void*)(reinterpret_cast<const char*>(ld.k) + base), (short)0, nbytes, 0x00020000);
@@ -585,9 +595,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const FlashParams p) 
 #pragma unroll
       for (int e = 0; e < 4; ++e) vreg[e] = Chunk::bload(vr, voff[e]);
     }
-    if constexpr (MASK) {
-      if (tid < BN) mreg = tid < ld.nvalid() ? p.mask[b * p.mask_bs + ld.key0 + tid] : 0.0f;
-    }
+    if (tid < BN) mreg = tid < ld.nvalid() ? p.mask[b * p.mask_bs + ld.key0 + tid] : 0.0f;
     ld.next(p);
   };
 
@@ -617,9 +625,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const FlashParams p) 
         *reinterpret_cast<uint2*>(vs + (vdc * 8 + 2 * w + 1) * VS + vkg * 4) = hi;
       }
     }
-    if constexpr (MASK) {
-      if (tid < BN) mask_s[buf][tid] = mreg;
-    }
+    if (tid < BN) mask_s[buf][tid] = mreg;
   };
 
   f32x16_t oacc[DB];
@@ -652,15 +658,6 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const FlashParams p) 
     const uint16_t* vs = ks + KBUF;
     const int nvalid = cp.nvalid();
 
-    // per-tile logit scale (and V scale for fp8)
-    float c_log2 = p.scale_log2;
-    float v_scale = 1.0f;
-    if constexpr (FP8) {
-      const int64_t f = cp.row0 / p.frame;
-      c_log2 *= p.k_sc[cp.s][b * p.sc_bs + h * p.sc_hs + f];
-      v_scale = p.v_sc[cp.s][b * p.sc_bs + h * p.sc_hs + f];
-    }
-
     // ---- S^T = K Q^T, fragments read one k-step ahead ----
     f32x16_t sacc[2] = {f32x16_t{}, f32x16_t{}};
     const uint16_t* kfrag = ks + li * KS + hg * 8;
@@ -684,15 +681,13 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const FlashParams p) 
     bf16x8_t vb = *reinterpret_cast<const bf16x8_t*>(vfrag + 16);
 
     // ---- online softmax on the accumulators (base-2 domain) ----
-    if constexpr (MASK) {
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int key = kb * 32 + 16 * (r >> 3) + 8 * hg + (r & 7);
-          sacc[kb][r] = fmaxf((sacc[kb][r] * p.scale + mask_s[buf][key]) * kLog2e, -3.0e38f);
-        }
-    }
+      for (int r = 0; r < 16; ++r) {
+        const int key = kb * 32 + 16 * (r >> 3) + 8 * hg + (r & 7);
+        sacc[kb][r] = fmaxf((sacc[kb][r] * p.scale + mask_s[buf][key]) * kLog2e, -3.0e38f);
+      }
     if (nvalid < BN) {
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
@@ -708,9 +703,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const FlashParams p) 
 #pragma unroll
       for (int r = 0; r < 16; ++r) mt = fmaxf(mt, sacc[kb][r]);
     mt = pair_max(mt);
-    // logits are x = s * c (c > 0), so max(x) = max(s) * c
-    const float c = MASK ? 1.0f : c_log2;
-    const float m_tile = mt * c;
+    const float m_tile = mt;
     const bool raise = m_tile > m_run + kLazy;
     if (__builtin_amdgcn_ballot_w64(raise)) {
       const float m_new = fmaxf(m_run, m_tile);
@@ -731,10 +724,10 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const FlashParams p) 
       uint32_t w[4];
 #pragma unroll
       for (int e = 0; e < 8; e += 2) {
-        const float p0 = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][8 * t + e], c, neg_m));
-        const float p1 = __builtin_amdgcn_exp2f(__builtin_fmaf(sacc[kb][8 * t + e + 1], c, neg_m));
+        const float p0 = __builtin_amdgcn_exp2f(sacc[kb][8 * t + e] + neg_m);
+        const float p1 = __builtin_amdgcn_exp2f(sacc[kb][8 * t + e + 1] + neg_m);
         psum += p0 + p1;
-        w[e >> 1] = FP8 ? pack_bf16x2(p0 * v_scale, p1 * v_scale) : pack_bf16x2(p0, p1);
+        w[e >> 1] = pack_bf16x2(p0, p1);
       }
       pf[ks4] = __builtin_bit_cast(bf16x8_t, make_uint4(w[0], w[1], w[2], w[3]));
     }
@@ -770,7 +763,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_kernel(const FlashParams p) 
 typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 // ---------------------------------------------------------------------------
-// Software-pipelined direct kernel (bf16; K token-major, V key-major in HBM).
+// Software-pipelined direct kernel (bf16; K token-major, V key- or token-major).
 //
 // What bounds it: power.  Under this kernel's random data the part clocks
 // down to 1.6-1.8 GHz: the 32x32x16 form of the kernel took 157 us (151-164 by box) at
@@ -798,9 +791,12 @@ typedef __attribute__((address_space(3))) void* lds_ptr_t;
 // 16*L), so no VGPRs and no VALU work go into staging.  Tile rows are not
 // padded; the chunks of a row are xor-swizzled (row_swizzle) and the K-row
 // order, the swizzle and the V transpose all happen in the address each lane
-// reads from.  V must be stored key-major (the KV arena's V layout); a
-// segment's last 8-token chunk is read whole and its keys past the segment
-// end are masked out of the softmax.
+// reads from.  V stored key-major (the KV arena's layout): a segment's last
+// 8-token chunk is read whole and its keys past the segment end are masked
+// out of the softmax.  V stored token-major (VTOK: plain cache tensors): its
+// tiles keep keys in rows and ds_read_b64_tr_b16 transposes the fragments, at
+// about 158 against 147 us at 1152 x 4608, where concatenating K and copying
+// V into a key-major store first took 105 us.
 //
 // The per-tile vector work is cut down and moved under the matrix cores:
 //
@@ -851,11 +847,12 @@ template <bool FRAMED>
 struct KeyStreamT {
   int s, rem, frem;
   int lim = 0x7FFFFFFF;  // keys past this index of the concatenated sequence are not part of the stream
+  int b = 0;             // batch row, times each segment's batch stride (0: the head offset holds it)
   const char* ptr;
   __device__ __forceinline__ void enter(const void* const* base, int64_t head, const FlashParams& p, int seg) {
     s = seg;
     rem = (int)((p.seg_start[seg + 1] < lim ? p.seg_start[seg + 1] : (int64_t)lim) - p.seg_start[seg]);
-    ptr = reinterpret_cast<const char*>(base[seg]) + head;
+    ptr = reinterpret_cast<const char*>(base[seg]) + (b * p.seg_bs[seg] + head);
     if constexpr (FRAMED) frem = p.frame;
   }
   __device__ __forceinline__ void seek(const void* const* base, int64_t head, int64_t tile_bytes,
@@ -911,7 +908,7 @@ struct KeyStreamT {
 // waves of a SIMD finish together, where two 4-wave workgroups on one CU do
 // not (the older one's waves win the issue arbitration and finish about a
 // quarter earlier, leaving the CU half busy until the other ends).
-template <int D, bool PAIR>
+template <int D, bool PAIR, bool VTOK>
 __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
   constexpr int BM = kBM, BN = kBN;
   constexpr int NKC = D / 8;         // 16-byte chunks of a K row
@@ -959,18 +956,20 @@ __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
   const int vrow_bytes = (int)(p.v_ds * 2);
   const int krow0 = (wave * 64 + lane) / NKC, vrow0 = (wave * 64 + lane) / NVC;
   const int kchunk = (lane % NKC) ^ row_swizzle<NKC>(krow0);
-  const int vchunk = (lane % NVC) ^ row_swizzle<NVC>(vrow0);
+  const int vchunk = VTOK ? (lane % NKC) ^ key_swizzle<NKC>(krow0) : (lane % NVC) ^ row_swizzle<NVC>(vrow0);
   const int koff = key_of_row(krow0) * row_bytes + kchunk * 16;
-  const int voff = vrow0 * vrow_bytes + vchunk * 16;
+  const int voff = (VTOK ? krow0 * row_bytes : vrow0 * vrow_bytes) + vchunk * 16;
   auto kslot_keys = [](int i) { return key_of_row(i * (256 / NKC)); };  // keys from slot 0's to slot i's
 
-  const int64_t k_head = (b * p.kv_bs + h * p.kv_hs) * 2;
-  const int64_t v_head = (b * p.v_bs + h * p.v_hs) * 2;
+  const int64_t k_head = h * p.kv_hs * 2;
+  const int64_t v_head = VTOK ? k_head : (b * p.v_bs + h * p.v_hs) * 2;
   const int64_t k_tile = (int64_t)BN * row_bytes;
-  const int64_t v_tile = BN * 2;
+  const int64_t v_tile = VTOK ? k_tile : BN * 2;
   KeyStreamT<false> kit, vit;
   kit.lim = klim;
   vit.lim = klim;
+  kit.b = b;
+  vit.b = VTOK ? b : 0;
   kit.seek(p.k_ptr, k_head, k_tile, p, wi.j0);
   vit.seek(p.v_ptr, v_head, v_tile, p, wi.j0);
   // LDS address of this wave's first load slot in a buffer; the empty asm
@@ -985,9 +984,9 @@ __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
   // tile's buffer range (a whole tile's is left open): those lanes load
   // zeros, and their scores are masked out of the softmax.  A whole tile's
   // slots take their uniform offset from a scalar register; a partial tile
-  // adds it per lane, so the range check sees the whole offset.  V (8-key
-  // chunks of key-major rows) re-reads the segment's last chunk for the
-  // positions past its end.
+  // adds it per lane, so the range check sees the whole offset.  Token-major V
+  // is bounded the same way; key-major V (8-key chunks of its rows) re-reads
+  // the segment's last chunk for the positions past its end.
   auto issue_k = [&](int buf) {
     const int nv = kit.nvalid();
     const uint32_t l0 = lds_slot0(kbuf + buf * KBUF);
@@ -1009,10 +1008,24 @@ __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
     kit.next(p.k_ptr, k_head, k_tile, p);
   };
   auto issue_v = [&](int buf) {
-    const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)vit.ptr, (short)0, 0x7FFFFFFF, 0x00020000);
     const uint32_t l0 = lds_slot0(vbuf + buf * VBUF);
     const int nv = vit.nvalid();
-    if (loader) {
+    if (VTOK && loader) {
+      const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)vit.ptr, (short)0,
+                                                        nv == BN ? 0x7FFFFFFF : nv * row_bytes, 0x00020000);
+      const bool whole = nv == BN;
+#pragma unroll
+      for (int i = 0; i < VSLOT; ++i) {
+        const int step = i * (256 / NKC) * row_bytes;
+        if (whole)
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(uintptr_t)(l0 + i * 4096), 16, voff, step, 0, 0);
+        else
+          __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(uintptr_t)(l0 + i * 4096), 16, voff + step, 0, 0,
+                                                   0);
+      }
+    }
+    if (!VTOK && loader) {
+      const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)vit.ptr, (short)0, 0x7FFFFFFF, 0x00020000);
       int off = voff;
       if (nv < BN) off = vrow0 * vrow_bytes + min(vchunk, (nv + 7) / 8 - 1) * 16;
 #pragma unroll
@@ -1096,8 +1109,24 @@ __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
   auto kfrag = [&](int buf, int kb, int s) -> bf16x8_t {
     return *reinterpret_cast<const bf16x8_t*>(kbuf + buf * KBUF + kb * 16 * D + (kofs ^ (s * 32)));
   };
+  // Token-major V tiles hold keys in rows, so a V^T fragment is read with the
+  // transposing LDS read: the 16 lanes of one lg read a block of 4 keys x 16
+  // channels (8 bytes per lane) and lane li receives its channel of the 4
+  // keys; two reads give the lane's 8 keys.
+  const int tofs = (8 * lg + (li >> 2)) * D + (((li >> 1) & 1) ^ key_swizzle<NKC>(8 * lg + (li >> 2))) * 8 +
+                   (li & 1) * 4;
   auto vfrag = [&](int buf, int d, int k2) -> bf16x8_t {
-    return *reinterpret_cast<const bf16x8_t*>(vbuf + buf * VBUF + d * 16 * BN + (vofs ^ (k2 * 32)));
+    if constexpr (VTOK) {
+      typedef short s16x4_t __attribute__((ext_vector_type(4)));
+      typedef short s16x8_t __attribute__((ext_vector_type(8)));
+      typedef __attribute__((address_space(3))) s16x4_t* lds_s16x4_t;
+      uint16_t* v0 = vbuf + buf * VBUF + 32 * k2 * D + (tofs ^ (16 * d));
+      const s16x4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)v0);
+      const s16x4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4_t)(v0 + 4 * D));
+      return __builtin_bit_cast(bf16x8_t, (s16x8_t)__builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+    } else {
+      return *reinterpret_cast<const bf16x8_t*>(vbuf + buf * VBUF + d * 16 * BN + (vofs ^ (k2 * 32)));
+    }
   };
   auto pfrag = [](const uint32_t (&pw)[16], int k2, int n) {
     const int q = 8 * k2 + 4 * n;
@@ -1153,7 +1182,7 @@ __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
   constexpr int NPV = 2 * CB, NS = NPV + 4 * KS;
   constexpr int PREF = 3;
   auto tile = [&](int vb, int kbf, const f32x4_t (&scur)[4][2], f32x4_t (&snext)[4][2], const uint32_t (&pprev)[16],
-                  uint32_t (&pcur)[16], float (&ps)[2], const float (&neg_m)[2]) {
+                  uint32_t (&pcur)[16], float (&ps)[2], const float (&neg_m)[2], auto&& loads) {
     auto frag = [&](int t) -> bf16x8_t {
       if (t < NPV) return vfrag(vb, t % CB, t / CB);
       return kfrag(kbf, (t - NPV) & 3, (t - NPV) >> 2);
@@ -1168,6 +1197,7 @@ __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
       if (t < NS) {
         if (t + PREF < NS) ring[(t + PREF) % (PREF + 1)] = frag(t + PREF);
         const bf16x8_t a = ring[t % (PREF + 1)];
+        if (VTOK && t == NPV - PREF) loads();
         // the query blocks alternate (0 1, 1 0, ...): consecutive MFMAs share an operand
 #pragma unroll
         for (int i = 0; i < 2; ++i) {
@@ -1229,7 +1259,10 @@ __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
       __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      if (VTOK && t + PREF < NPV)
+        __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+      else
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
       __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -1265,13 +1298,19 @@ __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
                     uint32_t (&pcur)[16]) {
       constexpr int jp = decltype(jpar)::value;
       publish();  // K(j+1) and V(j-1) have landed; the buffers of K(j) and V(j-2) are free
-      if (j + 2 < ntiles) issue_k(jp);  // K(j+2)
-      const int nv = vit.nvalid();      // valid keys of tile j
-      issue_v(jp);                      // V(j)
+      const int nv = vit.nvalid();  // valid keys of tile j
+      auto loads = [&]() {
+        if (j + 2 < ntiles) issue_k(jp);  // K(j+2)
+        issue_v(jp);                      // V(j)
+      };
+      // Token-major V: after the tile's last V fragment read instead (the
+      // compiler waits for every load to LDS in flight before a transposing
+      // read: 178 us with the loads here, at 1152 x 4608).
+      if (!VTOK) loads();
       if (nv < BN) mask_tail(scur, nv);
       const float neg_m[2] = {-m_run[0], -m_run[1]};
       float ps[2];
-      tile(1 - jp, 1 - jp, scur, snext, pprev, pcur, ps, neg_m);
+      tile(1 - jp, 1 - jp, scur, snext, pprev, pcur, ps, neg_m, loads);
       if (__builtin_amdgcn_ballot_w64(fmaxf(ps[0], ps[1]) > kOver)) {
         // raise m to the tile maximum, rescale O and l, redo P(j) from S(j)
 #pragma unroll
@@ -1354,9 +1393,10 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
   const int ntiles = wi.j1 > wi.j0 ? wi.j1 - wi.j0 : 0;
 
   const int row_bytes = (int)p.kv_ls;
-  const int64_t kv_head = b * p.kv_bs + h * p.kv_hs;
+  const int64_t kv_head = h * p.kv_hs;
   const int64_t kv_tile = (int64_t)BN * row_bytes;
   KeyStreamT<FRAMED> kit, vit;
+  kit.b = vit.b = b;
   kit.seek(p.k_ptr, kv_head, kv_tile, p, wi.j0);
   vit.seek(p.v_ptr, kv_head, kv_tile, p, wi.j0);
   // ---- register staging of the next K and V tiles ----
@@ -1720,22 +1760,25 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
   finish_tile<D>(p, wi, b, h, qt, owave * 32 + (int)(threadIdx.x & 31), oacc, m_run, pair_sum(l_run), stage);
 }
 
-template <int D, bool FP8>
+// KV operands of a kernel instance: bf16 with key-major V, bf16 with
+// token-major V, or fp8 (frames of whole 64-key tiles)
+enum KvKind { kKeyMajorV, kTokenMajorV, kFp8 };
+
+template <int D, KvKind KV>
 __global__ void __launch_bounds__(256, 2) flash_fwd_pipe_kernel(const FlashParams p) {
-  if constexpr (FP8)
+  if constexpr (KV == kFp8)
     flash_fp8_body<D, false>(p);
   else
-    flash_bf16_body<D, false>(p);
+    flash_bf16_body<D, false, KV == kTokenMajorV>(p);
 }
 
-// bf16 key-major V, or fp8 K/V in frames of whole 64-key tiles, with an even
-// number of q-tiles per head: pair workgroups
-template <int D, bool FP8>
+// an even number of q-tiles per head: pair workgroups
+template <int D, KvKind KV>
 __global__ void __launch_bounds__(512, 1) flash_fwd_pair_kernel(const FlashParams p) {
-  if constexpr (FP8)
+  if constexpr (KV == kFp8)
     flash_fp8_body<D, false, true>(p);
   else
-    flash_bf16_body<D, true>(p);
+    flash_bf16_body<D, true, KV == kTokenMajorV>(p);
 }
 
 // fp8 frames that are not a whole number of 64-key tiles
@@ -1761,26 +1804,26 @@ inline int64_t grid_blocks(const FlashParams& p) {
   return p.n_full + (nq - p.n_full) * p.split;
 }
 
-template <int D, bool FP8, bool FRAMED = false>
+template <int D, KvKind KV, bool FRAMED = false>
 int launch_flash_pipe(const FlashParams& p, hipStream_t st) {
-  static_assert(FP8 || !FRAMED, "frame tiling is an fp8 feature");
+  static_assert(KV == kFp8 || !FRAMED, "frame tiling is an fp8 feature");
   const int64_t nblocks = grid_blocks(p);
   LTX_REQUIRE(nblocks <= 0x7FFFFFFF, "ltx_flash_attn_fwd: grid too large");
   if constexpr (FRAMED)
     hipLaunchKernelGGL((flash_fwd_pipe_framed_kernel<D>), dim3((unsigned)nblocks), dim3(256), 0, st, p);
   else if (p.pair)
-    hipLaunchKernelGGL((flash_fwd_pair_kernel<D, FP8>), dim3((unsigned)nblocks), dim3(512), 0, st, p);
+    hipLaunchKernelGGL((flash_fwd_pair_kernel<D, KV>), dim3((unsigned)nblocks), dim3(512), 0, st, p);
   else
-    hipLaunchKernelGGL((flash_fwd_pipe_kernel<D, FP8>), dim3((unsigned)nblocks), dim3(256), 0, st, p);
+    hipLaunchKernelGGL((flash_fwd_pipe_kernel<D, KV>), dim3((unsigned)nblocks), dim3(256), 0, st, p);
   LTX_LAUNCH_CHECK("ltx_flash_attn_fwd");
   return launch_combine<D>(p, st);
 }
 
-template <int D, bool FP8, bool MASK>
-int launch_flash(const FlashParams& p, hipStream_t st) {
+template <int D>
+int launch_flash_masked(const FlashParams& p, hipStream_t st) {
   const int64_t nblocks = grid_blocks(p);
   LTX_REQUIRE(nblocks <= 0x7FFFFFFF, "ltx_flash_attn_fwd: grid too large");
-  hipLaunchKernelGGL((flash_fwd_kernel<D, FP8, MASK>), dim3((unsigned)nblocks), dim3(256), 0, st, p);
+  hipLaunchKernelGGL((flash_fwd_masked_kernel<D>), dim3((unsigned)nblocks), dim3(256), 0, st, p);
   LTX_LAUNCH_CHECK("ltx_flash_attn_fwd");
   return launch_combine<D>(p, st);
 }
@@ -1861,31 +1904,33 @@ inline int64_t workspace_bytes_for(int64_t tail, int split, int64_t D) {
 
 inline int64_t round256(int64_t x) { return (x + 255) / 256 * 256; }
 
-// Resident slots of the kernel a call with head size D takes: for
-// key-major bf16 V (vkey) the pair kernel when the q-tiles per head are
-// even (pair), else the pipelined kernel; for fp8 K/V the same choice (the
-// framed kernel shares the pipelined kernel's occupancy); else the staged
-// kernel (its masked instance for a key mask).
-inline Slots flash_slots(int64_t D, bool vkey, bool fp8, bool mask, bool pair) {
-  Slots s;
-  if (D == 128)
-    s = vkey && pair ? resident_slots<flash_fwd_pair_kernel<128, false>>(512)
-        : vkey       ? resident_slots<flash_fwd_pipe_kernel<128, false>>()
-        : fp8 && pair ? resident_slots<flash_fwd_pair_kernel<128, true>>(512)
-        : fp8        ? resident_slots<flash_fwd_pipe_kernel<128, true>>()
-        : mask       ? resident_slots<flash_fwd_kernel<128, false, true>>()
-                     : resident_slots<flash_fwd_kernel<128, false, false>>();
-  else
-    s = vkey && pair ? resident_slots<flash_fwd_pair_kernel<64, false>>(512)
-        : vkey       ? resident_slots<flash_fwd_pipe_kernel<64, false>>()
-        : fp8 && pair ? resident_slots<flash_fwd_pair_kernel<64, true>>(512)
-        : fp8        ? resident_slots<flash_fwd_pipe_kernel<64, true>>()
-        : mask       ? resident_slots<flash_fwd_kernel<64, false, true>>()
-                     : resident_slots<flash_fwd_kernel<64, false, false>>();
-  // pieces: one per CU for the pipelined kernels (and the pair kernel, one
-  // workgroup per CU), one per slot for the staged kernel (plan_split)
-  if (!vkey && !fp8) s.pieces = s.slots;
-  return s;
+// The kernel family a call takes: the masked staged kernel for a key mask,
+// else the pipelined one of its KV kind (the pair instance when the q-tiles
+// per head are even; fp8 framed shares the pipelined kernel's occupancy).
+enum FlashPath { kPathKeyMajor, kPathTokenMajor, kPathFp8, kPathMasked };
+
+template <int D>
+Slots slots_for(FlashPath path, bool pair) {
+  switch (path) {
+    case kPathKeyMajor:
+      return pair ? resident_slots<flash_fwd_pair_kernel<D, kKeyMajorV>>(512)
+                  : resident_slots<flash_fwd_pipe_kernel<D, kKeyMajorV>>();
+    case kPathTokenMajor:
+      return pair ? resident_slots<flash_fwd_pair_kernel<D, kTokenMajorV>>(512)
+                  : resident_slots<flash_fwd_pipe_kernel<D, kTokenMajorV>>();
+    case kPathFp8:
+      return pair ? resident_slots<flash_fwd_pair_kernel<D, kFp8>>(512)
+                  : resident_slots<flash_fwd_pipe_kernel<D, kFp8>>();
+    default: {
+      // pieces: one per slot for the staged kernel, one per CU for the others (plan_split)
+      Slots s = resident_slots<flash_fwd_masked_kernel<D>>();
+      s.pieces = s.slots;
+      return s;
+    }
+  }
+}
+inline Slots flash_slots(int64_t D, FlashPath path, bool pair) {
+  return D == 128 ? slots_for<128>(path, pair) : slots_for<64>(path, pair);
 }
 
 // fp8 K/V in frames of whole 64-key tiles with an odd number (>= 3) of
@@ -1908,11 +1953,11 @@ inline SplitPlan plan_fp8_split_launch(int64_t B, int64_t H, int64_t nqt, int nt
   SplitPlan sp{};
   // launch 0: pair units over the first nqt - 1 q-tiles of every head
   const int64_t nu0 = B * H * (nqt - 1) / 2;
-  plan_split(nu0, ntiles, flash_slots(D, false, true, false, true), &sp.n_full[0], &sp.split[0]);
+  plan_split(nu0, ntiles, flash_slots(D, kPathFp8, true), &sp.n_full[0], &sp.split[0]);
   sp.bytes[0] = sp.split[0] > 1 ? workspace_bytes_for((nu0 - sp.n_full[0]) * 2, sp.split[0], D) : 0;
   // launch 1: the last q-tile of every head, one piece per slot
   const int64_t nu1 = B * H;
-  const Slots s1 = flash_slots(D, false, true, false, false);
+  const Slots s1 = flash_slots(D, kPathFp8, false);
   sp.n_full[1] = nu1;
   sp.split[1] = 1;
   if (s1.slots > 0 && nu1 < s1.slots) {
@@ -1942,16 +1987,16 @@ extern "C" int ltx_flash_attn_workspace_size(int64_t B, int64_t Lq, int64_t H, i
   const int64_t nq = B * H * nqt;
   const bool pair = nqt % 2 == 0;
   int64_t need = 0;
-  // kernels: staged, pipelined (key-major V), fp8 pipelined (framed or
-  // not), fp8 pair (frames of whole tiles), masked staged
+  // (fp8 in frames that are not whole tiles takes single q-tiles at an even
+  // count too)
   for (int k = 0; k < 5; ++k) {
-    const bool vk = k == 1, f8 = k == 2 || k == 3, mk = k == 4;
-    const bool kp = (k == 1 || k == 3) && pair;
+    const FlashPath path = k == 4 ? kPathFp8 : (FlashPath)k;
+    const bool kp = pair && k != 4 && path != kPathMasked;
     const int64_t nu = kp ? nq / 2 : nq;
     int64_t n_full;
     int split;
     // with an unbounded key count the planned split is the largest any call of this shape plans
-    plan_split(nu, 1 << 30, flash_slots(D, vk, f8, mk, kp), &n_full, &split);
+    plan_split(nu, 1 << 30, flash_slots(D, path, kp), &n_full, &split);
     const int64_t b = split > 1 ? workspace_bytes_for((nu - n_full) * (kp ? 2 : 1), split, D) : 0;
     need = b > need ? b : need;
   }
@@ -1967,7 +2012,8 @@ extern "C" int ltx_flash_attn_workspace_size(int64_t B, int64_t Lq, int64_t H, i
 // The body of both attention entry points.  `strict_ws`: a planned split
 // whose partials do not fit the workspace is an error (the no-allocation
 // entry point, whose workspace is the fixed scratch array) instead of a
-// fallback to whole q-tiles.
+// fallback to whole q-tiles.  `seg_bs`: each segment's own batch stride (in
+// elements, instead of k_bs), for token-major bf16 K/V.
 static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, int64_t D,
                                int64_t q_bs, int64_t q_ls, int64_t q_hs, int64_t n_segments,
                                const void* const* k_ptrs, const void* const* v_ptrs,
@@ -1977,7 +2023,8 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
                                int64_t sc_bs, int64_t sc_hs, int64_t frame_tokens,
                                const float* key_mask, int64_t mask_bs, const int64_t* key_lens, void* out,
                                int64_t o_bs, int64_t o_ls, int64_t o_hs, float* lse, float scale,
-                               void* workspace, int64_t workspace_bytes, bool strict_ws, void* stream) {
+                               void* workspace, int64_t workspace_bytes, bool strict_ws, void* stream,
+                               const int64_t* seg_bs = nullptr) {
   LTX_REQUIRE(q && out, "ltx_flash_attn_fwd: null q/out");
   LTX_REQUIRE(D == 64 || D == 128, "ltx_flash_attn_fwd: head dim %lld unsupported (64 or 128)",
               (long long)D);
@@ -2015,7 +2062,7 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
   p.q_bs = q_bs; p.q_ls = q_ls; p.q_hs = q_hs;
   p.o_bs = o_bs; p.o_ls = o_ls; p.o_hs = o_hs;
   p.o_al16 = ((uintptr_t)out % 16 == 0 && o_bs % 8 == 0 && o_ls % 8 == 0 && o_hs % 8 == 0) ? 1 : 0;
-  p.kv_bs = k_bs; p.kv_ls = k_ls; p.kv_hs = k_hs;
+  p.kv_ls = k_ls; p.kv_hs = k_hs;
   p.v_bs = v_bs; p.v_hs = v_hs; p.v_ds = v_ds;
   p.sc_bs = sc_bs; p.sc_hs = sc_hs;
   p.mask_bs = mask_bs;
@@ -2041,6 +2088,10 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
       p.k_sc[n] = k_scales[i];
       p.v_sc[n] = v_scales[i];
     }
+    const int64_t bs = seg_bs != nullptr ? seg_bs[i] : k_bs;
+    LTX_REQUIRE((bs * esz) % 16 == 0, "ltx_flash_attn_fwd: segment %lld's batch stride must keep 16-byte rows",
+                (long long)i);
+    p.seg_bs[n] = bs * esz;
     p.k_ptr[n] = k_ptrs[i];
     p.v_ptr[n] = v_ptrs[i];
     p.seg_start[n + 1] = p.seg_start[n] + seg_lens[i];
@@ -2106,26 +2157,27 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
           lp[i].part_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + sp.off[i]);
           lp[i].part_o = reinterpret_cast<uint16_t*>(lp[i].part_ml + tail * sp.split[i] * kBM * 2);
         }
-        const int rc = D == 128 ? launch_flash_pipe<128, true>(lp[i], st) : launch_flash_pipe<64, true>(lp[i], st);
+        const int rc = D == 128 ? launch_flash_pipe<128, kFp8>(lp[i], st) : launch_flash_pipe<64, kFp8>(lp[i], st);
         if (rc != LTX_OK) return rc;
       }
       return LTX_OK;
     }
   }
   // balanced tail (needs a workspace; without one every q-tile runs whole).
-  // Key-major bf16 V, or fp8 K/V in frames of whole 64-key tiles, with an
+  // Without a key mask (and, for fp8 K/V, in frames of whole 64-key tiles) an
   // even number of q-tiles per head runs the pair kernel, whose grid counts
   // units of two q-tiles (two partial results per split unit).
+  const FlashPath path = key_mask != nullptr ? kPathMasked : fp8 ? kPathFp8 : vkey ? kPathKeyMajor : kPathTokenMajor;
   {
     const int64_t nq = (int64_t)B * H * p.n_qtiles;
     LTX_REQUIRE(nq <= 0x7FFFFFFF, "ltx_flash_attn_fwd: grid too large");
-    p.pair = (vkey || (fp8 && frame_tokens % kBN == 0)) && p.n_qtiles % 2 == 0 ? 1 : 0;
+    p.pair = path != kPathMasked && (!fp8 || frame_tokens % kBN == 0) && p.n_qtiles % 2 == 0 ? 1 : 0;
     const int64_t nu = p.pair ? nq / 2 : nq;
     const int per_unit = p.pair ? 2 : 1;
     int64_t n_full = nu;
     int split = 1;
     if (workspace != nullptr) {
-      plan_split(nu, p.tile_start[n], flash_slots(D, vkey, fp8, key_mask != nullptr, p.pair != 0), &n_full,
+      plan_split(nu, p.tile_start[n], flash_slots(D, path, p.pair != 0), &n_full,
                  &split);
       if (split > 1 && workspace_bytes_for((nu - n_full) * per_unit, split, D) > workspace_bytes) {
         LTX_REQUIRE(!strict_ws,
@@ -2145,26 +2197,19 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
       p.part_o = reinterpret_cast<uint16_t*>(p.part_ml + tail * split * kBM * 2);
     }
   }
-  if (vkey) {
-    if (D == 128) return launch_flash_pipe<128, false>(p, st);
-    return launch_flash_pipe<64, false>(p, st);
-  }
-  if (fp8) {
-    // the framed instances share the plain ones' occupancy (same registers
-    // and LDS), so the split plan above holds for them too
-    if (frame_tokens % kBN != 0) {
-      if (D == 128) return launch_flash_pipe<128, true, true>(p, st);
-      return launch_flash_pipe<64, true, true>(p, st);
-    }
-    if (D == 128) return launch_flash_pipe<128, true>(p, st);
-    return launch_flash_pipe<64, true>(p, st);
-  }
-  if (D == 128) {
-    if (key_mask) return launch_flash<128, false, true>(p, st);
-    return launch_flash<128, false, false>(p, st);
-  } else {
-    if (key_mask) return launch_flash<64, false, true>(p, st);
-    return launch_flash<64, false, false>(p, st);
+  switch (path) {
+    case kPathKeyMajor:
+      return D == 128 ? launch_flash_pipe<128, kKeyMajorV>(p, st) : launch_flash_pipe<64, kKeyMajorV>(p, st);
+    case kPathTokenMajor:
+      return D == 128 ? launch_flash_pipe<128, kTokenMajorV>(p, st) : launch_flash_pipe<64, kTokenMajorV>(p, st);
+    case kPathFp8:
+      // the framed instances share the plain ones' occupancy (same registers
+      // and LDS), so the split plan above holds for them too
+      if (frame_tokens % kBN != 0)
+        return D == 128 ? launch_flash_pipe<128, kFp8, true>(p, st) : launch_flash_pipe<64, kFp8, true>(p, st);
+      return D == 128 ? launch_flash_pipe<128, kFp8>(p, st) : launch_flash_pipe<64, kFp8>(p, st);
+    default:
+      return D == 128 ? launch_flash_masked<128>(p, st) : launch_flash_masked<64>(p, st);
   }
 }
 
@@ -2183,6 +2228,19 @@ extern "C" int ltx_flash_attn_fwd(const void* q, int64_t B, int64_t Lq, int64_t 
                              k_ls, k_hs, v_bs, v_ls, v_hs, v_ds, kv_dtype, k_scales, v_scales, sc_bs, sc_hs,
                              frame_tokens, key_mask, mask_bs, key_lens, out, o_bs, o_ls, o_hs, lse, scale,
                              workspace, workspace_bytes, false, stream);
+}
+
+extern "C" int ltx_flash_attn_fwd_plain(const void* q, int64_t B, int64_t Lq, int64_t H, int64_t D, int64_t q_bs,
+                                        int64_t q_ls, int64_t q_hs, int64_t n_segments, const void* const* k_ptrs,
+                                        const void* const* v_ptrs, const int64_t* seg_lens, const int64_t* seg_bs,
+                                        int64_t kv_ls, int64_t kv_hs, void* out, int64_t o_bs, int64_t o_ls,
+                                        int64_t o_hs, float* lse, float scale, void* workspace,
+                                        int64_t workspace_bytes, void* stream) {
+  clear_error();
+  LTX_REQUIRE(n_segments == 0 || seg_bs != nullptr, "ltx_flash_attn_fwd_plain: null segment batch strides");
+  return flash_attn_fwd_impl(q, B, Lq, H, D, q_bs, q_ls, q_hs, n_segments, k_ptrs, v_ptrs, seg_lens, 0, kv_ls, kv_hs,
+                             0, kv_ls, kv_hs, 1, LTX_BF16, nullptr, nullptr, 0, 0, 0, nullptr, 0, nullptr, out, o_bs,
+                             o_ls, o_hs, lse, scale, workspace, workspace_bytes, false, stream, seg_bs);
 }
 
 // ---------------------------------------------------------------------------

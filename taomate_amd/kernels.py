@@ -285,13 +285,16 @@ class KVSegment:
 def flash_attn(q: torch.Tensor, segments: List[KVSegment], out: torch.Tensor,
                key_mask: Optional[torch.Tensor] = None, lse: Optional[torch.Tensor] = None,
                scale: Optional[float] = None, frame_tokens: int = 0, noalloc: bool = False,
-               key_lens: Optional[Sequence[int]] = None) -> None:
+               key_lens: Optional[Sequence[int]] = None, segment_batch_strides: bool = False) -> None:
     """ltx_flash_attn_fwd.  q/out [B, Lq, H, D] bf16; key_mask float32 [B, Lk] additive.
     ``key_lens`` (B host ints): batch row b attends keys [0, key_lens[b]) only
     (a prefix-per-row padding mask, bf16 key-major V, on the pipelined kernel).
     ``noalloc`` calls ltx_flash_attn_fwd_noalloc instead: no workspace tensor,
     the split partials go to the library's fixed per-device scratch array
-    (calls overlapping on one device race on it)."""
+    (calls overlapping on one device race on it).
+    ``segment_batch_strides``: token-major bf16 segments may be separate
+    tensors whose batch strides differ (ltx_flash_attn_fwd_plain), with no
+    mask, key counts or ``noalloc``."""
     _need_gpu(q, out, key_mask, lse)
     if q.dtype != torch.bfloat16 or out.dtype != torch.bfloat16:
         raise TypeError("flash_attn: q and out must be bf16")
@@ -321,8 +324,10 @@ def flash_attn(q: torch.Tensor, segments: List[KVSegment], out: torch.Tensor,
         vs = (s.v.stride(0), s.v.stride(1), s.v.stride(2), s.v.stride(3))
         if kst is None:
             kst, vst = ks, vs
-        elif ks != kst or vs != vst:
+        elif (ks != kst or vs != vst) if not segment_batch_strides else (ks[1:] != kst[1:] or vs[1:] != vst[1:]):
             raise ValueError("flash_attn: all K/V segments must share strides")
+        if segment_batch_strides and (ks != vs[:3] or vs[3] != 1 or kv_code != N.BF16):
+            raise ValueError("flash_attn: segment_batch_strides takes token-major bf16 K and V of equal strides")
         if s.v.shape[1] != s.k.shape[1]:
             raise ValueError("flash_attn: k/v segment lengths differ")
         lk += s.k.shape[1]
@@ -349,6 +354,8 @@ def flash_attn(q: torch.Tensor, segments: List[KVSegment], out: torch.Tensor,
         mask_bs = 0 if key_mask.shape[0] == 1 else key_mask.stride(0)
     if lse is not None and (lse.dtype != torch.float32 or lse.shape != (B, H, Lq) or not lse.is_contiguous()):
         raise ValueError("flash_attn: lse must be contiguous float32 [B, H, Lq]")
+    if segment_batch_strides and (key_mask is not None or key_lens is not None or noalloc):
+        raise ValueError("flash_attn: segment_batch_strides takes no mask, key counts or noalloc")
     kl = None
     if key_lens is not None:
         if len(key_lens) != B or any(not 0 <= int(n) <= lk for n in key_lens):
@@ -357,6 +364,15 @@ def flash_attn(q: torch.Tensor, segments: List[KVSegment], out: torch.Tensor,
     kp = N.ptr_array([s.k.data_ptr() for s in segs])
     vp = N.ptr_array([s.v.data_ptr() for s in segs])
     lens = N.i64_array([s.k.shape[1] for s in segs])
+    if segment_batch_strides:
+        seg_bs = N.i64_array([s.k.stride(0) for s in segs])
+        ws, ws_bytes = _flash_workspace(q, B, Lq, H, D)
+        N.call("ltx_flash_attn_fwd_plain", q.data_ptr(), B, Lq, H, D, q.stride(0), q.stride(1), q.stride(2),
+               len(segs), ctypes.cast(kp, ctypes.c_void_p), ctypes.cast(vp, ctypes.c_void_p),
+               ctypes.cast(lens, ctypes.c_void_p), ctypes.cast(seg_bs, ctypes.c_void_p), kst[1], kst[2],
+               out.data_ptr(), out.stride(0), out.stride(1), out.stride(2), _ptr(lse),
+               float(scale) if scale is not None else 0.0, _ptr(ws), ws_bytes, _stream(q))
+        return
     ksp = N.ptr_array([s.k_scales.data_ptr() for s in segs]) if fp8 else None
     vsp = N.ptr_array([s.v_scales.data_ptr() for s in segs]) if fp8 else None
     args = (q.data_ptr(), B, Lq, H, D, q.stride(0), q.stride(1), q.stride(2),
