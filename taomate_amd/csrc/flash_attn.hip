@@ -1350,30 +1350,37 @@ __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
   finish_rows<D>(p, wi, b, h, qt, wave * 32, oacc, m_run, l_tot, smem + owave * 32 * D);
 }
 
-// The fp8 kernels' body.  FRAMED: frames that are not a whole number of 64-key
-// tiles, cut at frame boundaries (KeyStreamT<true>, its own kernel); frames of
-// 64k tokens take the plain tiling, which never crosses a frame either and
-// keeps the hot kernel's scalar state and registers as they were (the framed
-// state costs the D = 128 instance register spills).
-template <int D, bool FRAMED, bool PAIR = false>
-__device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
-  static_assert(!(PAIR && FRAMED), "pair workgroups take the plain tiling");
+// The 32x32x16 body: the fp8 kernels, and bf16 key-major V where the part is
+// not power bound (small_grid).  FRAMED (fp8 only): frames that are not a whole
+// number of 64-key tiles, cut at frame boundaries (KeyStreamT<true>, its own
+// kernel); frames of 64k tokens take the plain tiling, which never crosses a
+// frame either and keeps the hot kernel's scalar state and registers as they
+// were (the framed state costs the D = 128 instance register spills).
+template <int D, bool FP8, bool FRAMED, bool PAIR = false>
+__device__ __forceinline__ void flash_mfma32_body(const FlashParams& p) {
+  static_assert(FP8 || !FRAMED, "frame tiling is an fp8 feature");
+  static_assert(!PAIR || (FP8 && !FRAMED), "pair workgroups: fp8 in the plain tiling");
   constexpr int BM = kBM, BN = kBN;
   constexpr int NKC = D / 8;
   constexpr int KS = D + 8;
   // V^T tile rows (one head-dim channel, BN keys = 8 chunks of 16 bytes):
-  // with D = 128 two rows share one pad chunk (17 chunks per pair), else each
-  // row has its own (9 chunks).  Either way 16 consecutive rows' same chunk
-  // covers 16 distinct 16-byte bank groups, so a fragment read is
-  // conflict-free.
-  constexpr bool VPAIR = D == 128;
+  // with D = 128 two rows share one pad chunk (17 chunks per pair, 17 load
+  // instructions per tile), else each row has its own (9 chunks).  Either
+  // way 16 consecutive rows' same chunk covers 16 distinct 16-byte bank
+  // groups, so a fragment read is conflict-free.
+  constexpr bool VPAIR = (D / 2) * 17 % 64 == 0;
   constexpr int VS = BN + 8;                      // row stride without pairing
   constexpr int VPS = 2 * BN + 8;                 // pair stride with pairing
   constexpr int KBUF = BN * KS;
   constexpr int VBUF = VPAIR ? (D / 2) * VPS : D * VS;
+  constexpr int KINS = BN * (NKC + 1) / 64;
+  constexpr int VINS = VPAIR ? (D / 2) * 17 / 64 : D * 9 / 64;
+  constexpr int KSLOT = (KINS + 3) / 4;
+  constexpr int VSLOT = (VINS + 3) / 4;
   constexpr int DB = D / 32;
   constexpr int QS = D / 16;
   constexpr float kOver = 65536.0f;  // largest per-lane tile sum kept without raising m
+  static_assert(BN * (NKC + 1) % 64 == 0 && (VPAIR || D * 9 % 64 == 0), "tile does not split into whole instructions");
   // element offset of V^T row r in a V buffer
   auto vrow = [](int r) { return VPAIR ? (r >> 1) * VPS + (r & 1) * BN : r * VS; };
 
@@ -1390,16 +1397,123 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
   const int lane = threadIdx.x & 63;
   const int li = lane & 31, hg = lane >> 5;
   const int qi = qt * BM + wave * 32 + li;
-  const int ntiles = wi.j1 > wi.j0 ? wi.j1 - wi.j0 : 0;
+  // a per-batch key count ends this row's key tiles early (the streams stop
+  // at it, so its last tile is partial and masked like a segment's last)
+  const int klim = (!FP8 && p.n_klen) ? p.klen[b] : 0x7FFFFFFF;
+  int jend = wi.j1;
+  if (!FP8 && p.n_klen) {
+    const int tb = tiles_below(p, klim);
+    jend = jend < tb ? jend : tb;
+  }
+  const int ntiles = jend > wi.j0 ? jend - wi.j0 : 0;
 
-  const int row_bytes = (int)p.kv_ls;
-  const int64_t kv_head = h * p.kv_hs;
-  const int64_t kv_tile = (int64_t)BN * row_bytes;
+  // ---- per-lane load offsets (bytes from a tile's first key), loop invariant ----
+  const int row_bytes = (int)(p.kv_ls * (FP8 ? 1 : 2));
+  const int vrow_bytes = (int)(p.v_ds * 2);
+  auto kpos = [&](int i, int& r, int& c) {
+    const int pch = (wave + 4 * i) * 64 + lane;
+    r = sig(pch / (NKC + 1));
+    c = pch % (NKC + 1);
+    c = c < NKC ? c : 0;
+  };
+  // the (channel, 16-byte chunk) load slot i of this lane fills; a pad slot
+  // re-reads a valid chunk
+  auto vpos = [&](int i, int& d, int& c) {
+    const int pch = (wave + 4 * i) * 64 + lane;
+    if constexpr (VPAIR) {
+      const int q = pch % 17;
+      d = 2 * (pch / 17) + (q < 16 ? q >> 3 : 0);
+      c = q < 16 ? (q & 7) : 0;
+    } else {
+      d = pch / 9;
+      d = d < D ? d : 0;
+      c = pch % 9;
+      c = c < 8 ? c : 0;
+    }
+  };
+  int koff[KSLOT], voff[VSLOT];
+#pragma unroll
+  for (int i = 0; i < KSLOT; ++i) {
+    int r, c;
+    kpos(i, r, c);
+    koff[i] = r * row_bytes + c * 16;
+  }
+#pragma unroll
+  for (int i = 0; i < VSLOT; ++i) {
+    int d, c;
+    vpos(i, d, c);
+    voff[i] = d * vrow_bytes + c * 16;
+  }
+
+  const int64_t k_head = h * p.kv_hs * (FP8 ? 1 : 2);
+  const int64_t v_head = FP8 ? k_head : (b * p.v_bs + h * p.v_hs) * 2;
+  const int64_t k_tile = (int64_t)BN * row_bytes;
+  const int64_t v_tile = FP8 ? k_tile : BN * 2;
   KeyStreamT<FRAMED> kit, vit;
-  kit.b = vit.b = b;
-  kit.seek(p.k_ptr, kv_head, kv_tile, p, wi.j0);
-  vit.seek(p.v_ptr, kv_head, kv_tile, p, wi.j0);
-  // ---- register staging of the next K and V tiles ----
+  kit.lim = klim;
+  vit.lim = klim;
+  kit.b = b;
+  vit.b = FP8 ? b : 0;
+  kit.seek(p.k_ptr, k_head, k_tile, p, wi.j0);
+  vit.seek(p.v_ptr, v_head, v_tile, p, wi.j0);
+  // LDS address of this wave's first load slot in a buffer; the empty asm
+  // keeps the compiler from holding every (buffer, slot) address in its own
+  // scalar register across the loop (they cost one s_add each instead)
+  auto lds_slot0 = [&](uint16_t* buf0) {
+    uint32_t a = (uint32_t)(uintptr_t)(lds_ptr_t)(buf0 + wave * 512);
+    asm volatile("" : "+s"(a));
+    return a;
+  };
+  // One load instruction ("slot" i of this wave) of a K or V tile.  rs is the
+  // tile's buffer resource, l0 this wave's first LDS chunk of the buffer and
+  // nv the tile's valid keys.  K rows past a segment's end lie outside the
+  // partial tile's buffer range (issue_k): those lanes load zeros, and their
+  // scores are masked out of the softmax.  V (8-key chunks of key-major rows)
+  // re-reads the segment's last chunk for the positions past its end.
+  auto k_load = [&](__amdgpu_buffer_rsrc_t rs, uint32_t l0, int i) {
+    if (i < KSLOT && wave + 4 * i < KINS)
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(uintptr_t)(l0 + i * 4096), 16, koff[i], 0, 0, 0);
+  };
+  auto v_load = [&](__amdgpu_buffer_rsrc_t rs, uint32_t l0, int nv, int i) {
+    if (i < VSLOT && wave + 4 * i < VINS) {
+      int off = voff[i];
+      if (nv < BN) {
+        int d, c;
+        vpos(i, d, c);
+        off = d * vrow_bytes + min(c, (nv + 7) / 8 - 1) * 16;
+      }
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(uintptr_t)(l0 + i * 4096), 16, off, 0, 0, 0);
+    }
+  };
+  auto rsrc = [&](const char* ptr) { return __builtin_amdgcn_make_buffer_rsrc((void*)ptr, (short)0, 0x7FFFFFFF, 0x00020000); };
+  // whole tiles (every tile but a segment's last) take one branch and issue
+  // their loads from the precomputed offsets; a K tile's buffer range ends at
+  // its last valid row (a whole tile's is left open), so the partial tile
+  // issues the same loads
+  auto issue_k = [&](int buf) {
+    const int nv = kit.nvalid();
+    const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)kit.ptr, (short)0, nv == BN ? 0x7FFFFFFF : nv * row_bytes,
+                                                      0x00020000);
+    const uint32_t l0 = lds_slot0(kbuf[buf]);
+#pragma unroll
+    for (int i = 0; i < KSLOT; ++i) k_load(rs, l0, i);
+    kit.next(p.k_ptr, k_head, k_tile, p);
+  };
+  auto issue_v = [&](int buf) {
+    const auto rs = rsrc(vit.ptr);
+    const uint32_t l0 = lds_slot0(vbuf[buf]);
+    const int nv = vit.nvalid();
+    if (nv == BN) {
+#pragma unroll
+      for (int i = 0; i < VSLOT; ++i) v_load(rs, l0, BN, i);
+    } else {
+#pragma unroll
+      for (int i = 0; i < VSLOT; ++i) v_load(rs, l0, nv, i);
+    }
+    vit.next(p.v_ptr, v_head, v_tile, p);
+  };
+
+  // ---- fp8: register staging of the next K and V tiles ----
   // K: thread t moves 8-code chunk t % NKC of rows t / NKC + FROWS * i.
   // V: thread t (< NVP) moves 8-channel chunk t / 16 of keys 4 * (t % 16) .. +3
   // and writes them transposed (4 keys of 8 channel rows); 16 consecutive
@@ -1414,13 +1528,13 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
   const int fvg = tid % 16, fvc = tid / 16;
   const bool fv_on = tid < NVP;
   const bool stage_k = !PAIR || grp == 0, stage_v = !PAIR || grp == 1;  // wave-uniform
-  uint2 kreg[FKL], vreg[4];
+  uint2 kreg[FP8 ? FKL : 1], vreg[FP8 ? 4 : 1];
   auto load_k8 = [&]() {
     if (!stage_k) return;
     const auto rs = __builtin_amdgcn_make_buffer_rsrc((void*)kit.ptr, (short)0, kit.nvalid() * row_bytes, 0x00020000);
 #pragma unroll
     for (int i = 0; i < FKL; ++i) kreg[i] = KVChunk<true>::bload(rs, (fkr + FROWS * i) * row_bytes + fkc * 8);
-    kit.next(p.k_ptr, kv_head, kv_tile, p);
+    kit.next(p.k_ptr, k_head, k_tile, p);
   };
   auto load_v8 = [&]() {
     if (!stage_v) return;
@@ -1429,7 +1543,7 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
 #pragma unroll
       for (int e = 0; e < 4; ++e) vreg[e] = KVChunk<true>::bload(rs, (fvg * 4 + e) * row_bytes + fvc * 8);
     }
-    vit.next(p.v_ptr, kv_head, kv_tile, p);
+    vit.next(p.v_ptr, v_head, v_tile, p);
   };
   auto store_k8_row = [&](int buf, int i) {
     if (!stage_k) return;
@@ -1440,18 +1554,20 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
     for (int i = 0; i < FKL; ++i) store_k8_row(buf, i);
   };
   auto store_v8_half = [&](int buf, int half) {
-    if (!stage_v || !fv_on) return;
-    const uint32_t d0 = half ? vreg[0].y : vreg[0].x, d1 = half ? vreg[1].y : vreg[1].x;
-    const uint32_t d2 = half ? vreg[2].y : vreg[2].x, d3 = half ? vreg[3].y : vreg[3].x;
-    // channels 4*half + {0, 1} and {2, 3} of keys (0, 1) and (2, 3)
-    const uint32_t k01a = __builtin_amdgcn_perm(d1, d0, 0x05010400u), k23a = __builtin_amdgcn_perm(d3, d2, 0x05010400u);
-    const uint32_t k01b = __builtin_amdgcn_perm(d1, d0, 0x07030602u), k23b = __builtin_amdgcn_perm(d3, d2, 0x07030602u);
-    const int r0 = fvc * 8 + 4 * half;
-    uint16_t* vb = &vbuf[buf][fvg * 4];
-    *reinterpret_cast<uint2*>(vb + vrow(r0)) = make_uint2(KVChunk<true>::pair(k01a, false), KVChunk<true>::pair(k23a, false));
-    *reinterpret_cast<uint2*>(vb + vrow(r0 + 1)) = make_uint2(KVChunk<true>::pair(k01a, true), KVChunk<true>::pair(k23a, true));
-    *reinterpret_cast<uint2*>(vb + vrow(r0 + 2)) = make_uint2(KVChunk<true>::pair(k01b, false), KVChunk<true>::pair(k23b, false));
-    *reinterpret_cast<uint2*>(vb + vrow(r0 + 3)) = make_uint2(KVChunk<true>::pair(k01b, true), KVChunk<true>::pair(k23b, true));
+    if constexpr (FP8) {   // vreg holds the four staged code chunks only in the fp8 instances
+      if (!stage_v || !fv_on) return;
+      const uint32_t d0 = half ? vreg[0].y : vreg[0].x, d1 = half ? vreg[1].y : vreg[1].x;
+      const uint32_t d2 = half ? vreg[2].y : vreg[2].x, d3 = half ? vreg[3].y : vreg[3].x;
+      // channels 4*half + {0, 1} and {2, 3} of keys (0, 1) and (2, 3)
+      const uint32_t k01a = __builtin_amdgcn_perm(d1, d0, 0x05010400u), k23a = __builtin_amdgcn_perm(d3, d2, 0x05010400u);
+      const uint32_t k01b = __builtin_amdgcn_perm(d1, d0, 0x07030602u), k23b = __builtin_amdgcn_perm(d3, d2, 0x07030602u);
+      const int r0 = fvc * 8 + 4 * half;
+      uint16_t* vb = &vbuf[buf][fvg * 4];
+      *reinterpret_cast<uint2*>(vb + vrow(r0)) = make_uint2(KVChunk<true>::pair(k01a, false), KVChunk<true>::pair(k23a, false));
+      *reinterpret_cast<uint2*>(vb + vrow(r0 + 1)) = make_uint2(KVChunk<true>::pair(k01a, true), KVChunk<true>::pair(k23a, true));
+      *reinterpret_cast<uint2*>(vb + vrow(r0 + 2)) = make_uint2(KVChunk<true>::pair(k01b, false), KVChunk<true>::pair(k23b, false));
+      *reinterpret_cast<uint2*>(vb + vrow(r0 + 3)) = make_uint2(KVChunk<true>::pair(k01b, true), KVChunk<true>::pair(k23b, true));
+    }
   };
   // V(j) to LDS: the codes are interleaved by key before decoding: one v_perm
   // puts channels c and c + 1 of keys 2i and 2i + 1 into one word, whose low
@@ -1464,13 +1580,17 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
   };
   // the tile the softmax works on: its valid keys and (fp8) its scales
   KeyStreamT<FRAMED> cit;
-  cit.seek(p.k_ptr, 0, 0, p, wi.j0);
+  if constexpr (FP8) cit.seek(p.k_ptr, 0, 0, p, wi.j0);
   struct TileScale { float c, off, inv; };  // logit scale, exponent offset log2 sv, 1 / sv
   auto tile_scale = [&]() -> TileScale {
-    const int64_t o = b * p.sc_bs + h * p.sc_hs + cit.row0(p) / p.frame;
-    const float sk = p.k_sc[cit.s][o];
-    const float sv = p.v_sc[cit.s][o];
-    return TileScale{p.scale_log2 * sk, __log2f(sv), 1.0f / sv};
+    if constexpr (FP8) {
+      const int64_t o = b * p.sc_bs + h * p.sc_hs + cit.row0(p) / p.frame;
+      const float sk = p.k_sc[cit.s][o];
+      const float sv = p.v_sc[cit.s][o];
+      return TileScale{p.scale_log2 * sk, __log2f(sv), 1.0f / sv};
+    } else {
+      return TileScale{p.scale_log2, 0.0f, 1.0f};
+    }
   };
 
   // ---- Q^T fragments, resident for the whole key loop ----
@@ -1552,11 +1672,16 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
             *reinterpret_cast<const bf16x8_t*>(vf + vrow(d * 32) + k4 * 16), pf, oacc[d], 0, 0, 0);
     }
   };
-  // Tiles reach LDS through ds_writes, which the barrier waits for; the loads
-  // in flight only fill registers that the next slot program decodes (the
-  // compiler waits for each before its use), so they stay in flight across
-  // the barrier: 194.5 -> 192.8 us at 1152 x 4608.
-  auto publish = [&]() { __syncthreads(); };
+  // bf16: the tile loads go straight to LDS and are counted by vmcnt, so
+  // they must land before the barrier publishes them.  fp8: the staged tiles
+  // reach LDS through ds_writes (the barrier waits for those), and the
+  // loads in flight only fill registers that the next slot program decodes
+  // (the compiler waits for each before its use), so they stay in flight
+  // across the barrier: 194.5 -> 192.8 us at 1152 x 4608.
+  auto publish = [&]() {
+    if constexpr (!FP8) asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+  };
 
   // ---- the slot program of one tile ----
   // NS matrix-core slots: PV(j-1) (4*DB MFMAs over vbuf[vb]) then S(j+1)
@@ -1671,44 +1796,66 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
     f32x16_t sa[2], sb[2];
     uint32_t pa[16], pb[16];  // P(j) of even / odd j
     // ---- prologue: S(0) sets m from its own maximum; P(0); S(1) ----
-    // K(0), V(0), K(1) decoded into LDS; K(2) and V(1) left in registers
-    const int nv0 = cit.nvalid();
-    load_k8();
-    load_v8();
-    load_q();
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    store_k8(0);
-    store_v8(0);
-    if (ntiles > 1) {
+    int nv0;
+    if constexpr (FP8) {
+      // K(0), V(0), K(1) decoded into LDS; K(2) and V(1) left in registers
+      nv0 = cit.nvalid();
       load_k8();
-      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-      store_k8(1);
       load_v8();
+      load_q();
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      store_k8(0);
+      store_v8(0);
+      if (ntiles > 1) {
+        load_k8();
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        store_k8(1);
+        load_v8();
+      }
+      if (ntiles > 2) load_k8();
+      publish();
+    } else {
+      issue_k(0);
+      if (ntiles > 1) issue_k(1);
+      nv0 = vit.nvalid();  // valid keys of tile 0 (the V stream is at tile j before V(j) is issued)
+      issue_v(0);
+      load_q();  // its latency overlaps the first tiles' loads
+      publish();
     }
-    if (ntiles > 2) load_k8();
-    publish();
     qk_tile(0, sa);
     if (nv0 < BN) mask_tail(sa, nv0);
     {
       const TileScale ts = tile_scale();
       m_run = tile_max(sa, ts.c);
       l_run = exp_all(sa, pa, ts.c, ts.off - m_run) * ts.inv;
-      cit.next(p.k_ptr, 0, 0, p);
+      if constexpr (FP8) cit.next(p.k_ptr, 0, 0, p);
     }
     if (ntiles > 1) qk_tile(1, sb);
     if (ntiles > 2) {
       __syncthreads();  // every wave is done with K(0)
-      store_k8(0);                   // K(2)
-      if (ntiles > 3) load_k8();     // K(3)
+      if constexpr (FP8) {
+        store_k8(0);                   // K(2)
+        if (ntiles > 3) load_k8();     // K(3)
+      } else {
+        issue_k(0);                    // K(2)
+      }
     }
     // ---- iteration j (1 <= j < ntiles): the slot program computes
     //      O += V(j-1)^T P(j-1), S(j+1) = K(j+1) Q^T and P(j) = 2^(S(j)c - m).
     //      On the last tile S(j+1) is computed from stale LDS and dropped. ----
     auto step = [&](int j, f32x16_t (&scur)[2], f32x16_t (&snext)[2], const uint32_t (&pprev)[16],
                     uint32_t (&pcur)[16]) {
-      // registers hold K(j+2) and V(j); LDS holds K(j+1) and V(j-1)
-      publish();  // the buffers of K(j) and V(j-2) are free
-      const int nv = cit.nvalid();
+      int nv;
+      if constexpr (FP8) {
+        // registers hold K(j+2) and V(j); LDS holds K(j+1) and V(j-1)
+        publish();  // the buffers of K(j) and V(j-2) are free
+        nv = cit.nvalid();
+      } else {
+        publish();  // K(j+1) and V(j-1) have landed; the buffers of K(j) and V(j-2) are free
+        if (j + 2 < ntiles) issue_k(j & 1);  // K(j+2)
+        nv = vit.nvalid();                   // valid keys of tile j
+        issue_v(j & 1);                      // V(j)
+      }
       if (nv < BN) mask_tail(scur, nv);
       const TileScale ts = tile_scale();
       float ps0, ps1;
@@ -1716,14 +1863,16 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
       // loads of K(j+3) and V(j+1) into the freed registers ride in the slot
       // program, under the matrix work of tile j
       tile((j - 1) & 1, (j + 1) & 1, scur, snext, pprev, pcur, ps0, ps1, ts.c, ts.off - m_run, [&](int t) {
+        if constexpr (FP8) {
 #pragma unroll
-        for (int i = 0; i < FKL; ++i)
-          if (t == kStageSlot0 + kStageStride * i && j + 2 < ntiles) store_k8_row(j & 1, i);  // K(j+2)
-        if (t == kStageSlot0 + kStageStride * FKL && j + 3 < ntiles) load_k8();               // K(j+3)
+          for (int i = 0; i < FKL; ++i)
+            if (t == kStageSlot0 + kStageStride * i && j + 2 < ntiles) store_k8_row(j & 1, i);  // K(j+2)
+          if (t == kStageSlot0 + kStageStride * FKL && j + 3 < ntiles) load_k8();               // K(j+3)
 #pragma unroll
-        for (int hh = 0; hh < 2; ++hh)
-          if (t == kStageSlot0 + kStageStride * (FKL + 1 + hh)) store_v8_half(j & 1, hh);     // V(j)
-        if (t == kStageSlot0 + kStageStride * (FKL + 3) && j + 1 < ntiles) load_v8();         // V(j+1)
+          for (int hh = 0; hh < 2; ++hh)
+            if (t == kStageSlot0 + kStageStride * (FKL + 1 + hh)) store_v8_half(j & 1, hh);     // V(j)
+          if (t == kStageSlot0 + kStageStride * (FKL + 3) && j + 1 < ntiles) load_v8();         // V(j+1)
+        }
       });
       float ps = (ps0 + ps1) * ts.inv;
       if (__builtin_amdgcn_ballot_w64(ps > kOver)) {
@@ -1737,7 +1886,7 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
         ps = exp_all(scur, pcur, ts.c, ts.off - m_run) * ts.inv;
       }
       l_run += ps;
-      cit.next(p.k_ptr, 0, 0, p);
+      if constexpr (FP8) cit.next(p.k_ptr, 0, 0, p);
     };
     int j = 1;
     for (; j + 1 < ntiles; j += 2) {
@@ -1760,14 +1909,14 @@ __device__ __forceinline__ void flash_fp8_body(const FlashParams& p) {
   finish_tile<D>(p, wi, b, h, qt, owave * 32 + (int)(threadIdx.x & 31), oacc, m_run, pair_sum(l_run), stage);
 }
 
-// KV operands of a kernel instance: bf16 with key-major V, bf16 with
-// token-major V, or fp8 (frames of whole 64-key tiles)
-enum KvKind { kKeyMajorV, kTokenMajorV, kFp8 };
+// KV operands of a kernel instance: bf16 with key-major V (kKeyMajorV32: on
+// 32x32x16 MFMAs), bf16 with token-major V, or fp8 (frames of whole 64-key tiles)
+enum KvKind { kKeyMajorV, kKeyMajorV32, kTokenMajorV, kFp8 };
 
 template <int D, KvKind KV>
 __global__ void __launch_bounds__(256, 2) flash_fwd_pipe_kernel(const FlashParams p) {
-  if constexpr (KV == kFp8)
-    flash_fp8_body<D, false>(p);
+  if constexpr (KV == kFp8 || KV == kKeyMajorV32)
+    flash_mfma32_body<D, KV == kFp8, false>(p);
   else
     flash_bf16_body<D, false, KV == kTokenMajorV>(p);
 }
@@ -1776,7 +1925,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_pipe_kernel(const FlashParam
 template <int D, KvKind KV>
 __global__ void __launch_bounds__(512, 1) flash_fwd_pair_kernel(const FlashParams p) {
   if constexpr (KV == kFp8)
-    flash_fp8_body<D, false, true>(p);
+    flash_mfma32_body<D, true, false, true>(p);
   else
     flash_bf16_body<D, true, KV == kTokenMajorV>(p);
 }
@@ -1784,7 +1933,7 @@ __global__ void __launch_bounds__(512, 1) flash_fwd_pair_kernel(const FlashParam
 // fp8 frames that are not a whole number of 64-key tiles
 template <int D>
 __global__ void __launch_bounds__(256, 2) flash_fwd_pipe_framed_kernel(const FlashParams p) {
-  flash_fp8_body<D, true>(p);
+  flash_mfma32_body<D, true, true>(p);
 }
 
 template <int D>
@@ -1811,8 +1960,8 @@ int launch_flash_pipe(const FlashParams& p, hipStream_t st) {
   LTX_REQUIRE(nblocks <= 0x7FFFFFFF, "ltx_flash_attn_fwd: grid too large");
   if constexpr (FRAMED)
     hipLaunchKernelGGL((flash_fwd_pipe_framed_kernel<D>), dim3((unsigned)nblocks), dim3(256), 0, st, p);
-  else if (p.pair)
-    hipLaunchKernelGGL((flash_fwd_pair_kernel<D, KV>), dim3((unsigned)nblocks), dim3(512), 0, st, p);
+  else if (KV != kKeyMajorV32 && p.pair)
+    hipLaunchKernelGGL((flash_fwd_pair_kernel<D, KV == kKeyMajorV32 ? kKeyMajorV : KV>), dim3((unsigned)nblocks), dim3(512), 0, st, p);
   else
     hipLaunchKernelGGL((flash_fwd_pipe_kernel<D, KV>), dim3((unsigned)nblocks), dim3(256), 0, st, p);
   LTX_LAUNCH_CHECK("ltx_flash_attn_fwd");
@@ -1880,26 +2029,84 @@ Slots resident_slots(int threads = 256) {
 // pieces of >= 2 key tiles, so its few workgroups spread over the CUs: V2A
 // 75 x 1152 16.0 -> 12.5 us, audio self-attention 75 x 675 14.2 -> 12.6 us.
 // Zero tail tiles: no split.
-inline void plan_split(int64_t nq, int ntiles, Slots s, int64_t* n_full, int* split) {
+//
+// The kernels that hold two workgroups per CU choose the split by split_cost:
+// with one piece per CU as the only rule, tails of more than half the CUs ran
+// whole.  Measured at 32 heads x 128, B = 2, bf16: 3 q-tiles per head (192
+// workgroups) over 10368 keys 191 us whole, 146 in two ranges; 5 per head
+// 252 and 225; 13 per head (a tail of 320) 518 and 486; over 4608 keys 84 and
+// 69, 113 and 109, 235 and 226; over 2048 keys and fewer whole is as fast and
+// stays.  The pair kernel's rule stays as it is: at 6, 12 and 14 q-tiles per
+// head its partly filled rounds measured no slower than any split (the CUs
+// that work run faster while others idle; the part is power bound).
+inline int64_t workspace_bytes_for(int64_t tail, int64_t split, int64_t D) {
+  return tail * split * kBM * (2 * 4 + D * 2);  // (max, sum) fp32 + bf16 O row
+}
+
+// No plan's partials exceed the no-allocation entry point's scratch array, so
+// both entry points plan alike.
+inline int split_limit(int64_t tail_qtiles, int64_t D) {
+  const int64_t n = LTX_NOALLOC_SCRATCH_BYTES / workspace_bytes_for(tail_qtiles, 1, D);
+  return (int)(n < kMaxSplit ? n : kMaxSplit);
+}
+
+// Time of `tail` q-tiles of `ntiles` key tiles in `sp` ranges each, in units
+// of a key tile's time with two workgroups on every CU.  A round of r
+// workgroups of t tiles takes t when every slot is filled, 0.75 t + a share
+// for the CUs with two when r is more than one per CU, and 0.57 t with one
+// per CU (0.43 t behind whole rounds, whose older workgroups end early and
+// free their slots); 2 per round for the pieces' prologue and epilogue, and
+// 2.5 + 0.002 per piece for the combine kernel (half as much again at D = 64,
+// whose tiles are shorter).
+inline float split_cost(int64_t tail, int sp, int ntiles, Slots s, bool after_full, int64_t D) {
+  const int64_t m = tail * sp, whole = m / s.slots, rem = m % s.slots;
+  const float t = (float)((ntiles + sp - 1) / sp), k = D == 64 ? 1.5f : 1.0f;
+  float c = (float)whole * (t + 2.0f * k);
+  if (rem > s.pieces)
+    c += t * (0.75f + 0.25f * (float)(rem - s.pieces) / (float)s.pieces) + 2.0f * k;
+  else if (rem > 0)
+    c += t * (after_full || whole > 0 ? 0.43f : 0.57f) + 2.0f * k;
+  return sp > 1 ? c + k * (2.5f + 0.002f * (float)m) : c;
+}
+
+inline void plan_split(int64_t nq, int ntiles, Slots s, int64_t D, int per_unit, int64_t* n_full, int* split) {
   *n_full = nq;
   *split = 1;
   const int slots = s.slots;
   if (slots <= 0 || nq % slots == 0) return;
   const int64_t full = (nq / slots) * slots;
   const int64_t tail = nq - full;
-  int sp = (int)(s.pieces / tail);
-  if (sp > kMaxSplit) sp = kMaxSplit;
   // pieces keep >= 4 key tiles behind a whole round, >= 2 when the grid is
   // a single partial round (its few workgroups would leave most CUs idle)
   const int min_tiles = full > 0 ? 4 : 2;
-  if (sp > ntiles / min_tiles) sp = ntiles / min_tiles;
+  int most = split_limit(tail * per_unit, D);
+  if (most > ntiles / min_tiles) most = ntiles / min_tiles;
+  int sp = 1;
+  if (slots == 2 * s.pieces) {
+    float best = split_cost(tail, 1, ntiles, s, full > 0, D);
+    for (int i = 2; i <= most; ++i) {
+      const float c = split_cost(tail, i, ntiles, s, full > 0, D);
+      if (c < 0.94f * best) {
+        best = c;
+        sp = i;
+      }
+    }
+  } else {
+    sp = (int)(s.pieces / tail);
+    sp = sp > most ? most : sp;
+  }
   if (sp < 2) return;
   *n_full = full;
   *split = sp;
 }
 
-inline int64_t workspace_bytes_for(int64_t tail, int split, int64_t D) {
-  return tail * split * kBM * (2 * 4 + D * 2);  // (max, sum) fp32 + bf16 O row
+// Partial bytes that plan_split may ask for, whatever the key count.
+inline int64_t split_bytes_bound(int64_t nq, Slots s, int64_t D, int per_unit) {
+  if (s.slots <= 0 || nq % s.slots == 0) return 0;
+  const int64_t tail = (nq % s.slots);
+  int64_t sp = split_limit(tail * per_unit, D);
+  if (s.slots != 2 * s.pieces && sp > s.pieces / tail) sp = s.pieces / tail;
+  return sp > 1 ? workspace_bytes_for(tail * per_unit, sp, D) : 0;
 }
 
 inline int64_t round256(int64_t x) { return (x + 255) / 256 * 256; }
@@ -1933,6 +2140,18 @@ inline Slots flash_slots(int64_t D, FlashPath path, bool pair) {
   return D == 128 ? slots_for<128>(path, pair) : slots_for<64>(path, pair);
 }
 
+// Key-major bf16 calls that keep the 32x32x16 kernel: the 4-wave kernel with
+// little more than one workgroup per CU, or fewer than 16 key tiles.  The CUs
+// then hold one wave per SIMD for much of the call, the part is not power
+// bound, and a wave issues half as many MFMAs: 32.7 against 35.5 us for 3
+// q-tiles per head over 2048 keys (B = 2, 32 heads x 128: 192 workgroups), 70.5
+// against 73.8 us for 5 over 4608 keys at 32 x 64 (320), and 26.0 against
+// 27.4 us for 9 over 832 keys.  With 448 workgroups the 16x16x32 kernel leads
+// again (126.9 against 130.2 us, 7 over 4608 keys).
+inline bool small_grid(const FlashParams& p, Slots s) {
+  return !p.pair && (p.tile_start[p.n_seg] < 16 || 4 * grid_blocks(p) <= 5 * (int64_t)s.pieces);
+}
+
 // fp8 K/V in frames of whole 64-key tiles with an odd number (>= 3) of
 // q-tiles per head runs as two launches: the first n_qtiles - 1 q-tiles of
 // every head as pair workgroups (each thread stages half of a K/V tile that
@@ -1953,7 +2172,7 @@ inline SplitPlan plan_fp8_split_launch(int64_t B, int64_t H, int64_t nqt, int nt
   SplitPlan sp{};
   // launch 0: pair units over the first nqt - 1 q-tiles of every head
   const int64_t nu0 = B * H * (nqt - 1) / 2;
-  plan_split(nu0, ntiles, flash_slots(D, kPathFp8, true), &sp.n_full[0], &sp.split[0]);
+  plan_split(nu0, ntiles, flash_slots(D, kPathFp8, true), D, 2, &sp.n_full[0], &sp.split[0]);
   sp.bytes[0] = sp.split[0] > 1 ? workspace_bytes_for((nu0 - sp.n_full[0]) * 2, sp.split[0], D) : 0;
   // launch 1: the last q-tile of every head, one piece per slot
   const int64_t nu1 = B * H;
@@ -1993,11 +2212,7 @@ extern "C" int ltx_flash_attn_workspace_size(int64_t B, int64_t Lq, int64_t H, i
     const FlashPath path = k == 4 ? kPathFp8 : (FlashPath)k;
     const bool kp = pair && k != 4 && path != kPathMasked;
     const int64_t nu = kp ? nq / 2 : nq;
-    int64_t n_full;
-    int split;
-    // with an unbounded key count the planned split is the largest any call of this shape plans
-    plan_split(nu, 1 << 30, flash_slots(D, path, kp), &n_full, &split);
-    const int64_t b = split > 1 ? workspace_bytes_for((nu - n_full) * (kp ? 2 : 1), split, D) : 0;
+    const int64_t b = split_bytes_bound(nu, flash_slots(D, path, kp), D, kp ? 2 : 1);
     need = b > need ? b : need;
   }
   // the two-launch fp8 plan for an odd q-tile count
@@ -2177,8 +2392,7 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
     int64_t n_full = nu;
     int split = 1;
     if (workspace != nullptr) {
-      plan_split(nu, p.tile_start[n], flash_slots(D, path, p.pair != 0), &n_full,
-                 &split);
+      plan_split(nu, p.tile_start[n], flash_slots(D, path, p.pair != 0), D, per_unit, &n_full, &split);
       if (split > 1 && workspace_bytes_for((nu - n_full) * per_unit, split, D) > workspace_bytes) {
         LTX_REQUIRE(!strict_ws,
                     "ltx_flash_attn_fwd_noalloc: this call's split partials need %lld bytes, more than the "
@@ -2199,6 +2413,8 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
   }
   switch (path) {
     case kPathKeyMajor:
+      if (small_grid(p, flash_slots(D, path, p.pair != 0)))
+        return D == 128 ? launch_flash_pipe<128, kKeyMajorV32>(p, st) : launch_flash_pipe<64, kKeyMajorV32>(p, st);
       return D == 128 ? launch_flash_pipe<128, kKeyMajorV>(p, st) : launch_flash_pipe<64, kKeyMajorV>(p, st);
     case kPathTokenMajor:
       return D == 128 ? launch_flash_pipe<128, kTokenMajorV>(p, st) : launch_flash_pipe<64, kTokenMajorV>(p, st);
