@@ -109,6 +109,39 @@ def load() -> ctypes.CDLL:
         return lib
 
 
+HOST_NAME = "_ltx_host.so"
+_host = None
+
+
+def host():
+    """The native call module (csrc/host_calls.cpp), loaded once and bound to
+    the library's entry points: the checks and calls behind ``kernels``."""
+    global _host
+    if _host is not None:
+        return _host
+    lib = load()
+    with _lock:
+        if _host is not None:
+            return _host
+        path = LIB_DIR / HOST_NAME
+        if not path.exists():
+            raise NativeLibraryError(
+                f"{path} is not built; run `python -c 'import __graft_entry__ as g; g.build()'` "
+                "or `python -m taomate_amd.build`")
+        import importlib.machinery
+        import importlib.util
+        import torch  # noqa: F401  (the module links against torch's libraries)
+        try:
+            loader = importlib.machinery.ExtensionFileLoader("_ltx_host", str(path))
+            mod = importlib.util.module_from_spec(importlib.util.spec_from_loader("_ltx_host", loader))
+            loader.exec_module(mod)
+        except ImportError as e:
+            raise NativeLibraryError(f"cannot load {path}: {e}") from e
+        mod.bind({n: ctypes.cast(getattr(lib, n), ctypes.c_void_p).value for n in SIGNATURES}, NativeCallError)
+        _host = mod
+        return mod
+
+
 def call(name: str, *args) -> None:
     """Invoke an entry point and raise NativeCallError on failure."""
     lib = load()

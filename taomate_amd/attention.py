@@ -79,11 +79,16 @@ class CausalLTXAttention(nn.Module):
             return None
         w, b = pk
         n = self.inner_dim
-        for i, lin in enumerate((self.to_q, self.to_k, self.to_v)):
-            if lin.weight.data_ptr() != w[i * n].data_ptr() or lin.bias is None or \
-                    lin.bias.data_ptr() != b[i * n:].data_ptr() or lin.weight.shape != w[i * n:(i + 1) * n].shape:
+        wp, bp, shape = w.data_ptr(), b.data_ptr(), (n, w.shape[1])
+        w_step, b_step = n * w.stride(0) * w.element_size(), n * b.element_size()
+        for name in ("to_q", "to_k", "to_v"):
+            lin = self._modules[name]._parameters
+            lw, lb = lin["weight"], lin["bias"]
+            if lw.data_ptr() != wp or lb is None or lb.data_ptr() != bp or lw.shape != shape:
                 self._qkv_packed = None   # a parameter was replaced: drop the stale buffer
                 return None
+            wp += w_step
+            bp += b_step
         return w, b
 
     def cache_text_kv_(self, enabled: bool = True, size: int = 4) -> "CausalLTXAttention":
@@ -195,11 +200,13 @@ def _norm_rope(attn: CausalLTXAttention, q_lin: torch.Tensor, k_lin: torch.Tenso
     q = torch.empty_like(q_lin)
     k = torch.empty_like(k_lin) if k_out is None else k_out
     kp = k_pe if k_pe is not None else pe
-    gq = attn.q_norm.weight if attn.q_norm.weight is not None else None
-    gk = attn.k_norm.weight if attn.k_norm.weight is not None else None
+    q_norm, k_norm = attn.q_norm, attn.k_norm
+    gq, gk, eq, ek = q_norm.weight, k_norm.weight, q_norm.eps, k_norm.eps
     _check_bf16(gq, gk)
-    eq = attn.q_norm.eps if attn.q_norm.eps is not None else torch.finfo(q_lin.dtype).eps
-    ek = attn.k_norm.eps if attn.k_norm.eps is not None else torch.finfo(k_lin.dtype).eps
+    if eq is None:
+        eq = torch.finfo(q_lin.dtype).eps
+    if ek is None:
+        ek = torch.finfo(k_lin.dtype).eps
     kernels.qk_rmsnorm_rope(q_lin, q, gq, eq, pe, H, D, k_lin, k, gk, ek, kp, v_in=v_in, v_out=v_out)
     return q, k
 
@@ -226,15 +233,11 @@ def _finish(attn: CausalLTXAttention, out: torch.Tensor, x: torch.Tensor) -> tor
     return attn.to_out(out)
 
 
-def _key_padding_mask(mask: Optional[torch.Tensor], B: int, Lk: int) -> Optional[torch.Tensor]:
-    """Reduce the reference's mask forms (flex_attention_utils.py:250-264) to the
-    additive float32 [B or 1, Lk] key mask the kernel takes.  Masks that vary
-    per query are not on the inference path."""
-    if mask is None:
-        return None
+def _key_mask_rows(mask: torch.Tensor, B: int, Lk: int) -> torch.Tensor:
+    """The reference's mask forms (flex_attention_utils.py:250-264) as a
+    [B or 1, Lk] view.  Masks that vary per query are not on the inference
+    path."""
     m = mask
-    if m.dtype == torch.bool:
-        m = torch.zeros(m.shape, dtype=torch.float32, device=m.device).masked_fill_(~m, float("-inf"))
     if m.ndim == 4:
         if m.shape[1] != 1 or m.shape[2] != 1:
             raise NotImplementedError("only key-padding masks [B,1,1,Lk] are supported")
@@ -250,7 +253,14 @@ def _key_padding_mask(mask: Optional[torch.Tensor], B: int, Lk: int) -> Optional
         raise NotImplementedError(f"mask of shape {tuple(mask.shape)}")
     if m.shape[-1] != Lk:
         raise ValueError(f"mask covers {m.shape[-1]} keys, attention has {Lk}")
-    return m.to(torch.float32).contiguous()
+    return m
+
+
+def _additive_mask(rows: torch.Tensor) -> torch.Tensor:
+    """The additive float32 key mask the kernel takes."""
+    if rows.dtype == torch.bool:
+        return torch.zeros(rows.shape, dtype=torch.float32, device=rows.device).masked_fill_(~rows, float("-inf"))
+    return rows.to(torch.float32).contiguous()
 
 
 # A key-padding mask whose kept keys are a prefix of each batch row, with
@@ -265,13 +275,15 @@ def _key_padding_mask(mask: Optional[torch.Tensor], B: int, Lk: int) -> Optional
 _PREFIX: Dict[int, Tuple[int, Optional[Tuple[int, ...]]]] = {}
 
 
-def _kept_prefixes(mask: torch.Tensor, km: torch.Tensor) -> Optional[Tuple[int, ...]]:
-    """Per mask row, the length of the kept prefix, when every row keeps a
-    non-empty prefix and drops the rest; else None."""
+def _kept_prefixes(mask: torch.Tensor, rows: torch.Tensor) -> Optional[Tuple[int, ...]]:
+    """Per row of the mask (``rows``: its key rows), the length of the kept
+    prefix, when every row keeps a non-empty prefix and drops the rest; else
+    None."""
     key = id(mask)
     hit = _PREFIX.get(key)
     if hit is not None and hit[0] == mask._version:
         return hit[1]
+    km = _additive_mask(rows)
     kept, dropped = km == 0, km <= -1e30
     n: Optional[Tuple[int, ...]] = None
     if bool((kept | dropped).all()):
@@ -318,21 +330,23 @@ def standard_attention_forward(q: torch.Tensor, k: torch.Tensor, v: torch.Tensor
         if kk.stride() != vv.stride():
             kk = kk.contiguous()
             vv = vv.contiguous()
-    km = _key_padding_mask(mask, B, k.shape[1])
-    key_lens = None
-    if km is not None:
-        lens = _kept_prefixes(mask, km)
+    km = key_lens = None
+    if mask is not None:
+        rows = _key_mask_rows(mask, B, k.shape[1])
+        lens = _kept_prefixes(mask, rows)
         if lens is not None and len(set(lens)) == 1:
             n = lens[0]
-            kk, vv, km = kk[:, :n], vv[:, :n], None
+            kk, vv = kk[:, :n], vv[:, :n]
         elif lens is not None and B <= N.MAX_KEYLEN_BATCH and D in (64, 128) and Lq >= 256:
             # prefixes of different lengths: per-row key counts on the pipelined
             # kernel (with fewer queries the masked kernel, whatever V's layout,
             # so a cached key-major V gives the same result as a fresh one)
-            key_lens, km = lens, None
+            key_lens = lens
             if not key_major:
                 vv = _key_major(vv)
                 key_major = True
+        else:   # the masked kernel; the float mask is only made for it
+            km = _additive_mask(rows)
     if km is not None and key_major:
         # the masked kernel reads token-major V with K's strides
         kk = kk.contiguous()

@@ -1,4 +1,4 @@
-"""Build recipe for libtaomate_ltx.so (hipcc, gfx950 only).
+"""Build recipe for libtaomate_ltx.so (hipcc, gfx950 only) and the native call module.
 
     python -m taomate_amd.build          # compiles every csrc/*.hip, links lib/libtaomate_ltx.so
 
@@ -17,6 +17,7 @@ PKG = pathlib.Path(__file__).resolve().parent
 CSRC = PKG / "csrc"
 BUILD = PKG / "_build"
 LIB = PKG / "lib" / "libtaomate_ltx.so"
+HOST = PKG / "lib" / "_ltx_host.so"   # csrc/host_calls.cpp: the Python module that checks and makes the calls
 ARCH = "gfx950"
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
@@ -42,6 +43,19 @@ def _run(cmd):
 PER_SOURCE = {"flash_attn.hip": ["-mllvm", "-pragma-unroll-threshold=200000"]}
 
 
+def _host_command(out: pathlib.Path):
+    """g++ line of the native call module, against this interpreter's Python and torch."""
+    import sysconfig
+    import torch
+    t = pathlib.Path(torch.__file__).resolve().parent
+    rocm = os.environ.get("ROCM_PATH", "/opt/rocm")
+    return ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__", "-DUSE_ROCM",
+            f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}",
+            f"-I{t / 'include'}", f"-I{rocm}/include", f"-I{sysconfig.get_paths()['include']}",
+            str(CSRC / "host_calls.cpp"), "-o", str(out),
+            f"-L{t / 'lib'}", "-ltorch_python", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+
+
 def build(verbose: bool = False) -> pathlib.Path:
     BUILD.mkdir(exist_ok=True)
     LIB.parent.mkdir(exist_ok=True)
@@ -52,6 +66,8 @@ def build(verbose: bool = False) -> pathlib.Path:
     for src in sources:
         obj = BUILD / (src.stem + ".o")
         jobs.append((obj, [HIPCC, *FLAGS, *PER_SOURCE.get(src.name, []), "-c", str(src), "-o", str(obj)]))
+    host_tmp = HOST.with_suffix(".so.tmp")
+    jobs.append((host_tmp, _host_command(host_tmp)))
     workers = min(len(jobs), max(1, (os.cpu_count() or 2) // 2))
     with cf.ThreadPoolExecutor(workers) as ex:
         outs = list(ex.map(lambda j: _run(j[1]), jobs))
@@ -60,7 +76,8 @@ def build(verbose: bool = False) -> pathlib.Path:
             if o.strip():
                 print(o)
     tmp = LIB.with_suffix(".so.tmp")
-    _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *[str(o) for o, _ in jobs]])
+    _run([HIPCC, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", str(tmp), *[str(o) for o, _ in jobs[:-1]]])
+    os.replace(host_tmp, HOST)
     os.replace(tmp, LIB)
     return LIB
 
