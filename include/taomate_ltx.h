@@ -300,6 +300,20 @@ int ltx_flash_attn_fwd_noalloc(const void* q, int64_t B, int64_t Lq, int64_t H, 
 int ltx_flash_attn_workspace_size(int64_t B, int64_t Lq, int64_t H, int64_t D, int64_t* bytes);
 
 /*
+ * A linear layer over a few rows: y = act(x) W^T + bias, bf16, float32 sums.
+ * Replaces the nn.Linear calls of the timestep embedding and modulation
+ * (ltx_causal/transformer/compat.py:150-275: TimestepEmbedding,
+ * AdaLayerNormSingle), one row per sample.
+ *   x [M, K] rows x_ls apart (M <= 8, K a multiple of 8, at most 4096), W [N, K]
+ *   rows w_ls apart, bias [N] or NULL, y [M, N] rows y_ls apart; x and W rows
+ *   16-byte aligned.  silu != 0 applies SiLU to x first (float32, rounded to
+ *   bf16).
+ */
+int ltx_skinny_linear(int64_t M, int64_t N, int64_t K, const void* x, int64_t x_ls, int silu,
+                      const void* w, int64_t w_ls, const void* bias, void* y, int64_t y_ls,
+                      void* stream);
+
+/*
  * Gated residual update and AdaLN-modulated RMSNorm, bf16 [B, L, C] rows.
  * Replaces the bf16 tensor-op chains of block_forward_with_cache
  * (ltx_causal/transformer/kv_cache.py:2194-2633) around each attention and

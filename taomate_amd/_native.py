@@ -60,6 +60,7 @@ SIGNATURES = {
     "ltx_flash_attn_fwd_plain": [_ptr, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _i64, _ptr, _ptr, _ptr, _ptr,
                                  _i64, _i64, _ptr, _i64, _i64, _i64, _ptr, _f32, _ptr, _i64, _ptr],
     "ltx_flash_attn_workspace_size": [_i64, _i64, _i64, _i64, _ptr],
+    "ltx_skinny_linear": [_i64, _i64, _i64, _ptr, _i64, _int, _ptr, _i64, _ptr, _ptr, _i64, _ptr],
     "ltx_adaln": [_i64, _i64, _i64, _ptr, _i64, _i64, _ptr, _i64, _i64, _ptr, _i64, _i64, _ptr, _i64, _i64,
                   _ptr, _i64, _i64, _ptr, _i64, _i64, _ptr, _i64, _i64, _f32, _ptr],
 }

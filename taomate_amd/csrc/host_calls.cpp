@@ -37,6 +37,7 @@ struct Api {
   decltype(&ltx_flash_attn_fwd_plain) flash_attn_fwd_plain;
   decltype(&ltx_flash_attn_workspace_size) flash_attn_workspace_size;
   decltype(&ltx_adaln) adaln;
+  decltype(&ltx_skinny_linear) skinny_linear;
 } api;
 PyObject* native_call_error = nullptr;  // taomate_amd._native.NativeCallError
 
@@ -461,6 +462,24 @@ void adaln(PyObject* const* a) {
        (float)real(a[7]), stream_of(x));
 }
 
+// -------------------------------------------------------------- skinny linear
+// (x, weight, bias, y, silu)
+void skinny_linear(PyObject* const* a) {
+  const at::Tensor &x = tensor(a[0]), &w = tensor(a[1]), &y = tensor(a[3]);
+  const Opt bias = optional(a[2]);
+  for (Opt t : {Opt(&x), Opt(&w), bias, Opt(&y)}) {
+    need_gpu(t);
+    if (t != nullptr && t->scalar_type() != at::kBFloat16) type_error("skinny_linear: every tensor must be bf16");
+  }
+  if (x.dim() != 2 || w.dim() != 2 || y.dim() != 2 || x.size(1) != w.size(1) || y.size(0) != x.size(0) ||
+      y.size(1) != w.size(0) || x.stride(1) != 1 || w.stride(1) != 1 || y.stride(1) != 1)
+    value_error("skinny_linear: x " + shape(x) + ", weight " + shape(w) + ", y " + shape(y));
+  if (bias != nullptr && (bias->dim() != 1 || bias->size(0) != w.size(0) || bias->stride(0) != 1))
+    value_error("skinny_linear: bias must be a contiguous [N] vector");
+  call("ltx_skinny_linear", api.skinny_linear, x.size(0), w.size(0), x.size(1), ptr(&x), x.stride(0),
+       (int)truth(a[4]), ptr(&w), w.stride(0), ptr(bias), ptr(&y), y.stride(0), stream_of(x));
+}
+
 // ------------------------------------------------------------------- bindings
 template <void (*Fn)(PyObject* const*), Py_ssize_t N>
 PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -500,6 +519,7 @@ PyObject* bind(PyObject*, PyObject* args) {
   get("ltx_flash_attn_fwd_plain", api.flash_attn_fwd_plain);
   get("ltx_flash_attn_workspace_size", api.flash_attn_workspace_size);
   get("ltx_adaln", api.adaln);
+  get("ltx_skinny_linear", api.skinny_linear);
   if (!ok) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind: missing entry point addresses");
     return nullptr;
@@ -515,6 +535,7 @@ PyMethodDef methods[] = {
     {"kv_append", (PyCFunction)(void*)&entry<kv_append, 4>, METH_FASTCALL, nullptr},
     {"kv_append_fp8_pair", (PyCFunction)(void*)&entry<kv_append_fp8_pair, 7>, METH_FASTCALL, nullptr},
     {"flash_attn", (PyCFunction)(void*)&entry<flash_attn, 10>, METH_FASTCALL, nullptr},
+    {"skinny_linear", (PyCFunction)(void*)&entry<skinny_linear, 5>, METH_FASTCALL, nullptr},
     {"adaln", (PyCFunction)(void*)&entry<adaln, 8>, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ltx_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};

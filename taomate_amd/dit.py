@@ -82,6 +82,21 @@ def timestep_embedding(t: torch.Tensor, dim: int = 256, max_period: int = 10000)
     return torch.cat([torch.cos(emb), torch.sin(emb)], dim=-1)
 
 
+def _row_linear(lin: nn.Module, x: torch.Tensor, act: Optional[nn.Module] = None) -> torch.Tensor:
+    """``lin(act(x))`` for a few rows (one per sample or frame): a plain bf16
+    nn.Linear without hooks reads its weight once (ltx_skinny_linear); anything
+    else runs as modules."""
+    if (type(lin) is nn.Linear and x.is_cuda and x.dtype == torch.bfloat16 and lin.weight.dtype == torch.bfloat16
+            and not torch.is_grad_enabled() and x.dim() == 2 and 1 <= x.shape[0] <= kernels.SKINNY_MAX_ROWS
+            and x.shape[1] <= kernels.SKINNY_MAX_K and x.shape[1] % 8 == 0
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+            and lin.weight.is_contiguous() and lin.weight.data_ptr() % 16 == 0 and lin.weight.device == x.device
+            and not (lin._forward_hooks or lin._forward_pre_hooks)
+            and (act is None or (type(act) is nn.SiLU and not (act._forward_hooks or act._forward_pre_hooks)))):
+        return kernels.skinny_linear(x, lin.weight, lin.bias, silu=act is not None)
+    return lin(x if act is None else act(x))
+
+
 class TimestepEmbedding(nn.Module):
     def __init__(self, in_channels: int, dim: int):
         super().__init__()
@@ -90,7 +105,7 @@ class TimestepEmbedding(nn.Module):
         self.linear_2 = nn.Linear(dim, dim)
 
     def forward(self, x: torch.Tensor) -> torch.Tensor:
-        return self.linear_2(self.act(self.linear_1(x)))
+        return _row_linear(self.linear_2, _row_linear(self.linear_1, x), self.act)
 
 
 class _CombinedEmbedding(nn.Module):
@@ -113,7 +128,7 @@ class AdaLayerNormSingle(nn.Module):
 
     def forward(self, t: torch.Tensor, dtype: torch.dtype) -> Tuple[torch.Tensor, torch.Tensor]:
         e = self.emb(t, dtype)
-        return self.linear(self.silu(e)), e
+        return _row_linear(self.linear, e, self.silu), e
 
 
 @dataclass

@@ -153,6 +153,18 @@ def flash_attn(q: torch.Tensor, segments: List[KVSegment], out: torch.Tensor,
                                      segment_batch_strides)
 
 
+SKINNY_MAX_ROWS, SKINNY_MAX_K = 8, 4096
+
+
+def skinny_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
+                  silu: bool = False) -> torch.Tensor:
+    """ltx_skinny_linear: act(x) @ weight.T + bias for x [M <= 8, K <= 4096]
+    bf16 (SiLU of x first with ``silu``); K must be a multiple of 8."""
+    y = torch.empty(x.shape[0], weight.shape[0], dtype=x.dtype, device=x.device)
+    (N._host or N.host()).skinny_linear(x, weight, bias, y, silu)
+    return y
+
+
 def adaln(x: torch.Tensor, y: Optional[torch.Tensor] = None, gate: Optional[torch.Tensor] = None,
           x_out: Optional[torch.Tensor] = None, n_out: Optional[torch.Tensor] = None,
           scale: Optional[torch.Tensor] = None, shift: Optional[torch.Tensor] = None, eps: float = 1e-6) -> None:
