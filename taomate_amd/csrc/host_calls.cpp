@@ -502,6 +502,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
 PyObject* bind(PyObject*, PyObject* args) {
   PyObject *dict, *error;
   if (!PyArg_ParseTuple(args, "O!O", &PyDict_Type, &dict, &error)) return nullptr;
+  Api next{};
   bool ok = true;
   auto get = [&](const char* name, auto& fn) {
     PyObject* o = PyDict_GetItemString(dict, name);
@@ -509,21 +510,22 @@ PyObject* bind(PyObject*, PyObject* args) {
     ok = ok && p != nullptr;
     fn = reinterpret_cast<std::remove_reference_t<decltype(fn)>>(p);
   };
-  get("ltx_last_error", api.last_error);
-  get("ltx_qk_rmsnorm_rope", api.qk_rmsnorm_rope);
-  get("ltx_qk_rmsnorm_rope_v", api.qk_rmsnorm_rope_v);
-  get("ltx_kv_append", api.kv_append);
-  get("ltx_kv_append_fp8_pair", api.kv_append_fp8_pair);
-  get("ltx_flash_attn_fwd", api.flash_attn_fwd);
-  get("ltx_flash_attn_fwd_noalloc", api.flash_attn_fwd_noalloc);
-  get("ltx_flash_attn_fwd_plain", api.flash_attn_fwd_plain);
-  get("ltx_flash_attn_workspace_size", api.flash_attn_workspace_size);
-  get("ltx_adaln", api.adaln);
-  get("ltx_skinny_linear", api.skinny_linear);
+  get("ltx_last_error", next.last_error);
+  get("ltx_qk_rmsnorm_rope", next.qk_rmsnorm_rope);
+  get("ltx_qk_rmsnorm_rope_v", next.qk_rmsnorm_rope_v);
+  get("ltx_kv_append", next.kv_append);
+  get("ltx_kv_append_fp8_pair", next.kv_append_fp8_pair);
+  get("ltx_flash_attn_fwd", next.flash_attn_fwd);
+  get("ltx_flash_attn_fwd_noalloc", next.flash_attn_fwd_noalloc);
+  get("ltx_flash_attn_fwd_plain", next.flash_attn_fwd_plain);
+  get("ltx_flash_attn_workspace_size", next.flash_attn_workspace_size);
+  get("ltx_adaln", next.adaln);
+  get("ltx_skinny_linear", next.skinny_linear);
   if (!ok) {
     if (!PyErr_Occurred()) PyErr_SetString(PyExc_ValueError, "bind: missing entry point addresses");
     return nullptr;
   }
+  api = next;
   Py_INCREF(error);
   Py_XSETREF(native_call_error, error);
   Py_RETURN_NONE;

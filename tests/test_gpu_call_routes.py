@@ -1,0 +1,136 @@
+"""Calls whose route depends on their form, each against the general path or a
+reference: plain caches in strides and alignments that are attended in place
+or concatenated, key-range splits of partly filled grids, norm rows without
+RoPE tables, and the timestep MLPs with and without the row kernel."""
+import math
+
+import pytest
+import torch
+
+import taomate_amd as T
+from taomate_amd import dit, kernels
+from taomate_amd.kernels import KVSegment
+
+from .helpers import gen, randn
+
+pytestmark = pytest.mark.gpu
+
+
+def _attend64(q, k, v):
+    s = torch.einsum("bqhd,bkhd->bhqk", q.double(), k.double()) / math.sqrt(q.shape[-1])
+    return torch.einsum("bhqk,bkhd->bqhd", s.softmax(-1), v.double())
+
+
+def _bound(v):
+    # P, the output and the ratio of the rounded P's to the row sum: half a bf16 ulp each
+    return 3 * 2.0 ** -9 * v.abs().max().item()
+
+
+def _odd_offset(t):
+    """The same values in storage that starts 2 bytes past a 16-byte boundary."""
+    s = torch.empty(t.numel() + 8, dtype=t.dtype, device=t.device)
+    return s[1:1 + t.numel()].view(t.shape).copy_(t)
+
+
+FORMS = {
+    "contiguous": lambda t: t.contiguous(),
+    "batch_slice": lambda t: torch.cat([t, t], 1)[:, :t.shape[1]],
+    "token_offset": lambda t: torch.cat([t.new_zeros(t.shape[0], 3, *t.shape[2:]), t], 1)[:, 3:],
+    "head_major": lambda t: t.permute(0, 2, 1, 3).contiguous().permute(0, 2, 1, 3),
+    "row_gap": lambda t: torch.cat([t, t], -1)[..., :t.shape[-1]],
+    "odd_offset": _odd_offset,
+}
+
+
+@pytest.mark.parametrize("B", [1, 2])
+@pytest.mark.parametrize("Lc,L", [(1, 5), (64, 130), (203, 300)])
+@pytest.mark.parametrize("kform,vform", [(f, f) for f in FORMS] + [("contiguous", "head_major"),
+                                                                 ("contiguous", "odd_offset"),
+                                                                 ("batch_slice", "contiguous")])
+def test_plain_cache_forms(dev, kform, vform, Lc, L, B):
+    """attention_with_cache over plain tensors: every cache form gives the
+    result of contiguous cache tensors within the kernels' bf16 rounding."""
+    H, D = 4, 64
+    g = gen(Lc + L)
+    attn = T.CausalLTXAttention(H * D, heads=H, dim_head=D)
+    with torch.no_grad():
+        for p in attn.parameters():
+            p.copy_(torch.randn(p.shape, generator=g) * 0.05)
+        attn = attn.to(dev, torch.bfloat16)
+        x = randn((B, L, H * D), g, torch.bfloat16).to(dev)
+        ck, cv = (randn((B, Lc, H, D), g, torch.bfloat16).to(dev) for _ in range(2))
+        want, wk, wv = T.attention_with_cache(attn, x, None, None, None, ck, cv)
+        out, nk, nv = T.attention_with_cache(attn, x, None, None, None, FORMS[kform](ck), FORMS[vform](cv))
+    torch.cuda.synchronize()
+    assert torch.equal(nk, wk) and torch.equal(nv, wv)
+    # two roundings of the attention output (2^-8 relative), through to_out
+    err = (out.float() - want.float()).norm() / want.float().norm()
+    assert err <= 2.0 ** -7, err.item()
+
+
+@pytest.mark.parametrize("layout", ["key", "token"])
+@pytest.mark.parametrize("B,H,D,qtiles,keys", [(2, 32, 64, 3, 4608), (2, 16, 128, 5, 2500), (1, 32, 64, 7, 3000),
+                                              (2, 32, 64, 11, 6001), (2, 8, 128, 1, 300)])
+def test_split_plans(dev, layout, B, H, D, qtiles, keys):
+    """Grids whose last round is partly filled: the planned key-range split
+    against float64 on some heads, and the same plan in the no-allocation
+    entry point bit for bit."""
+    Lq = qtiles * 128 - 37
+    g = torch.Generator(device=dev)
+    g.manual_seed(keys)
+    r = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+    q, k = r(B, Lq, H, D), r(B, keys, H, D)
+    v = r(B, H, D, -(-keys // 8) * 8).permute(0, 3, 1, 2)[:, :keys] if layout == "key" else r(B, keys, H, D)
+    out, again = torch.empty_like(q), torch.empty_like(q)
+    lse = torch.empty(B, H, Lq, dtype=torch.float32, device=dev)
+    kernels.flash_attn(q, [KVSegment(k, v)], out, lse=lse)
+    kernels.flash_attn(q, [KVSegment(k, v)], again, noalloc=True)
+    torch.cuda.synchronize()
+    assert torch.equal(out, again)
+    for h in (0, H - 1):
+        sl = slice(h, h + 1)
+        ref = _attend64(q[:, :, sl].cpu(), k[:, :, sl].cpu(), v[:, :, sl].cpu())
+        assert (out[:, :, sl].double().cpu() - ref).abs().max().item() <= _bound(v) + 2.0 ** -8 * ref.abs().max().item()
+
+
+@pytest.mark.parametrize("B,L,H,D", [(2, 1, 8, 64), (1, 33, 32, 128), (2, 75, 32, 64)])
+def test_norm_without_tables(dev, B, L, H, D):
+    """Rows with a norm and a gain but no RoPE tables (the branch-free form)
+    equal the rotated form under identity tables bit for bit, also from packed
+    q/k/v columns and on one side alone."""
+    g = gen(L)
+    n = H * D
+    y = randn((B, L, 3 * n), g, torch.bfloat16).to(dev)
+    gq, gk = (randn((n,), g, torch.bfloat16).to(dev) for _ in range(2))
+    eye = (torch.ones(1, H, L, D // 2, dtype=y.dtype, device=dev), torch.zeros(1, H, L, D // 2, dtype=y.dtype, device=dev))
+    got, want = ([torch.empty(B, L, n, dtype=y.dtype, device=dev) for _ in range(3)] for _ in range(2))
+    for out, tab in ((got, None), (want, eye)):
+        kernels.qk_rmsnorm_rope(y[..., :n], out[0], gq, 1e-6, tab, H, D, y[..., n:2 * n], out[1], gk, 1e-6, tab)
+        kernels.qk_rmsnorm_rope(y[..., :n], out[2], gq, 1e-6, tab, H, D)
+    torch.cuda.synchronize()
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)
+    assert torch.equal(got[0], got[2])
+
+
+@pytest.mark.parametrize("rows", [1, 2, 6, 8, 9])
+def test_timestep_mlp_routes(dev, rows):
+    """AdaLayerNormSingle without grad (the row kernel up to 8 rows) against
+    the module path that grad mode, a hook or a replaced activation takes."""
+    m = dit.AdaLayerNormSingle(512, 6).to(dev, torch.bfloat16)
+    g = gen(rows)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.copy_((torch.randn(p.shape, generator=g) * 0.05).to(dev))
+    t = (torch.rand(rows, generator=g) * 1000).to(dev)
+    with torch.no_grad():
+        out, e = m(t, torch.bfloat16)
+    want, we = (z.detach() for z in m(t, torch.bfloat16))
+    for a, b in ((out, want), (e, we)):   # a few bf16 roundings through three layers
+        assert a.shape == b.shape and ((a - b).float().norm() / b.float().norm()).item() <= 2.0 ** -6
+    seen = []
+    h = m.linear.register_forward_hook(lambda *_: seen.append(1))
+    with torch.no_grad():
+        m(t, torch.bfloat16)
+    h.remove()
+    assert seen == [1]
