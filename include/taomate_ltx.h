@@ -275,11 +275,10 @@ int ltx_flash_attn_fwd_plain(const void* q, int64_t B, int64_t Lq, int64_t H, in
  *   sufficient workspace; the split partials go to a fixed device array of
  *   LTX_NOALLOC_SCRATCH_BYTES inside the library (one per device, kept until
  *   the process ends).  Allocates nothing: no hipMalloc / hipFree, no
- *   allocating library call.  A call whose split would need more scratch
- *   than that returns LTX_EINVAL with a message (at most two partial
- *   results per CU, 512 x 128 rows x (8 + 2 D) bytes, are ever planned on
- *   MI355X: 17.3 MB for D = 128).  Calls that overlap in time on one device share the
- *   array and race: serialise them (one stream, or events).
+ *   allocating library call.  Both entry points plan splits whose partials fit
+ *   that array, so the results are the same.  Calls that overlap in time on
+ *   one device share the array and race: serialise them (one stream, or
+ *   events).
  */
 #define LTX_NOALLOC_SCRATCH_BYTES (24ll << 20)
 int ltx_flash_attn_fwd_noalloc(const void* q, int64_t B, int64_t Lq, int64_t H, int64_t D,

@@ -2042,7 +2042,13 @@ Slots resident_slots(int threads = 256) {
 // workgroups) over 10368 keys 191 us whole, 146 in two ranges; 5 per head
 // 252 and 225; 13 per head (a tail of 320) 518 and 486; over 4608 keys 84 and
 // 69, 113 and 109, 235 and 226; over 2048 keys and fewer whole is as fast and
-// stays.  The pair kernel's rule stays as it is: at 6, 12 and 14 q-tiles per
+// stays.  The search starts at one piece per CU and only goes finer: fewer,
+// longer pieces average out less of their bf16 partials' rounding.  With the
+// count free, 98 of 264 grids of 75 to 300 queries over 330 to 2600 keys had a
+// larger error against float64 than one piece per CU gives (by up to 1.9 %),
+// with this floor none has.  75 x 675 at 32 x 64, B = 1, takes 13.0 -> 11.4 us
+// with it (token-major V); 300 x 330 at 16 x 64, B = 2, is 1.24 times as long
+// as whole.  The pair kernel's rule stays as it is: at 6, 12 and 14 q-tiles per
 // head its partly filled rounds measured no slower than any split (the CUs
 // that work run faster while others idle; the part is power bound).
 inline int64_t workspace_bytes_for(int64_t tail, int64_t split, int64_t D) {
@@ -2087,19 +2093,18 @@ inline void plan_split(int64_t nq, int ntiles, Slots s, int64_t D, int per_unit,
   const int min_tiles = full > 0 ? 4 : 2;
   int most = split_limit(tail * per_unit, D);
   if (most > ntiles / min_tiles) most = ntiles / min_tiles;
-  int sp = 1;
+  int sp = (int)(s.pieces / tail);
+  sp = sp > most ? most : sp;
+  sp = sp < 1 ? 1 : sp;
   if (slots == 2 * s.pieces) {
-    float best = split_cost(tail, 1, ntiles, s, full > 0, D);
-    for (int i = 2; i <= most; ++i) {
+    float best = split_cost(tail, sp, ntiles, s, full > 0, D);
+    for (int i = sp + 1; i <= most; ++i) {
       const float c = split_cost(tail, i, ntiles, s, full > 0, D);
       if (c < 0.94f * best) {
         best = c;
         sp = i;
       }
     }
-  } else {
-    sp = (int)(s.pieces / tail);
-    sp = sp > most ? most : sp;
   }
   if (sp < 2) return;
   *n_full = full;
@@ -2469,13 +2474,11 @@ extern "C" int ltx_flash_attn_fwd_plain(const void* q, int64_t B, int64_t Lq, in
 // No-allocation variant: the split partials live in a fixed device array.
 //
 // `scratch` holds the partial results of the split tail q-tiles (per piece:
-// 128 rows of (max, sum) in float32 and an O row in bf16).  The partial
-// results are at most two per CU (pieces <= resident slots, two 4-wave
-// workgroups per CU; the pair kernel's units hold two q-tiles at one
-// workgroup per CU), so a launch needs at most 2 CUs x 128 x (8 + 2 D) bytes:
-// 17.3 MB for D = 128 at 256 CUs (the fp8 two-launch plan keeps both
-// launches' partials in the array and is taken only when they fit).  Every piece writes its whole partial before the
-// combine kernel reads it, so nothing needs clearing between calls.  Each
+// 128 rows of (max, sum) in float32 and an O row in bf16).  split_limit keeps
+// every plan's partials within the array (the fp8 two-launch plan keeps both
+// launches' partials in it and is taken only when they fit).  Every piece
+// writes its whole partial before the combine kernel reads it, so nothing
+// needs clearing between calls.  Each
 // device holds its own copy of the array for the life of the process; its
 // device address is looked up once per device (hipGetSymbolAddress) and
 // only that address is handed to kernels.  Calls that overlap in time on one
