@@ -18,6 +18,7 @@
 
 #include <map>
 #include <mutex>
+#include <optional>
 #include <string>
 #include <utility>
 #include <vector>
@@ -89,7 +90,10 @@ struct Ref {
     if (p == nullptr) throw Refused{nullptr, ""};
   }
   Ref(Ref&& r) noexcept : o(std::exchange(r.o, nullptr)) {}
-  Ref(const Ref&) = delete;
+  Ref& operator=(Ref&& r) noexcept {
+    std::swap(o, r.o);
+    return *this;
+  }
   ~Ref() { Py_XDECREF(o); }
 };
 
@@ -134,17 +138,20 @@ Rows rows(const at::Tensor& t, int64_t hd) {
   return {t.size(1), t.stride(0), t.stride(1)};
 }
 
+// cos and sin point into `pair`, which may be the only holder of its items (a
+// table given as one stacked tensor or an iterator): it lives as long as they do.
 struct Table {
+  std::optional<Ref> pair;
   Opt cos = nullptr, sin = nullptr;
   int64_t tb = 0, th = 0, tt = 0;
 };
 Table table(PyObject* o, int64_t H, int64_t D, int64_t L, int64_t B) {
   Table r;
   if (o == Py_None) return r;
-  Ref seq(PySequence_Fast(o, "a RoPE table is a (cos, sin) pair"));
-  if (PySequence_Fast_GET_SIZE(seq.o) != 2) value_error("a RoPE table is a (cos, sin) pair");
-  r.cos = &tensor(PySequence_Fast_GET_ITEM(seq.o, 0));
-  r.sin = &tensor(PySequence_Fast_GET_ITEM(seq.o, 1));
+  PyObject* seq = r.pair.emplace(PySequence_Fast(o, "a RoPE table is a (cos, sin) pair")).o;
+  if (PySequence_Fast_GET_SIZE(seq) != 2) value_error("a RoPE table is a (cos, sin) pair");
+  r.cos = &tensor(PySequence_Fast_GET_ITEM(seq, 0));
+  r.sin = &tensor(PySequence_Fast_GET_ITEM(seq, 1));
   const at::Tensor &c = *r.cos, &s = *r.sin;
   if (c.sizes() != s.sizes() || c.strides() != s.strides() || c.scalar_type() != s.scalar_type())
     value_error("cos/sin tables must share shape, strides and dtype");

@@ -113,6 +113,24 @@ def test_norm_without_tables(dev, B, L, H, D):
     assert torch.equal(got[0], got[2])
 
 
+@pytest.mark.parametrize("form", ["list", "stacked", "iterator"])
+def test_table_forms(dev, form):
+    """A RoPE table given as a list, one stacked tensor or an iterator (whose
+    items only the call holds) rotates as the (cos, sin) tuple does."""
+    B, L, H, D = 2, 19, 4, 64
+    g = gen(3)
+    y = randn((B, L, H * D), g, torch.bfloat16).to(dev)
+    gain = randn((H * D,), g, torch.bfloat16).to(dev)
+    pair = torch.stack([randn((1, H, L, D // 2), g, torch.bfloat16) for _ in range(2)]).to(dev)
+    forms = {"tuple": lambda: (pair[0], pair[1]), "list": lambda: [pair[0], pair[1]], "stacked": lambda: pair,
+             "iterator": lambda: (t.clone() for t in pair)}
+    got, want = ([torch.empty_like(y) for _ in range(2)] for _ in range(2))
+    for out, f in ((got, form), (want, "tuple")):
+        kernels.qk_rmsnorm_rope(y, out[0], gain, 1e-6, forms[f](), H, D, y, out[1], gain, 1e-6, forms[f]())
+    torch.cuda.synchronize()
+    assert all(torch.equal(a, b) for a, b in zip(got, want))
+
+
 @pytest.mark.parametrize("rows", [1, 2, 6, 8, 9])
 def test_timestep_mlp_routes(dev, rows):
     """AdaLayerNormSingle without grad (the row kernel up to 8 rows) against

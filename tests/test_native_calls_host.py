@@ -1,7 +1,10 @@
 """The native call module's argument checks, without a GPU: what the wrappers
-refuse and with which error."""
+refuse and with which error, and how long they hold what they are given."""
+import weakref
+
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 
 from taomate_amd import _native, kernels
 from taomate_amd.kernels import KVSegment
@@ -33,3 +36,45 @@ def test_wrong_objects_raise_python_errors():
         host.bind({}, RuntimeError)
     with pytest.raises(ValueError, match="device tensors"):   # the refused bind left the calls bound
         kernels.adaln(x, n_out=x)
+
+
+class _OwnTables:
+    """A (cos, sin) argument that nothing but its iteration holds."""
+
+    def __init__(self):
+        self.refs = []
+
+    def __iter__(self):
+        for _ in range(2):
+            t = torch.ones(1, 1, 4, 32)
+            self.refs.append(weakref.ref(t))
+            yield t
+
+
+class _Eps:
+    """An eps that is read after the tables, and records whether they are still there."""
+
+    def __init__(self, tables):
+        self.tables, self.alive = tables, []
+
+    def __float__(self):
+        self.alive += [r() is not None for r in self.tables.refs]
+        return 1e-6
+
+
+@pytest.mark.parametrize("side", ["q", "k"])
+def test_rope_tables_are_held_for_the_call(side):
+    """The call reads the tables long after it took them apart: a pair that the
+    caller does not hold (an iterator's, a stacked tensor's rows) stays alive.
+    A device tensor without storage stands for the rows; the call ends at its
+    missing data pointer."""
+    with FakeTensorMode():
+        rows = torch.empty(1, 4, 64, dtype=torch.bfloat16, device="cuda")
+    tab = _OwnTables()
+    eps = _Eps(tab)
+    q_tab, k_tab = (tab, None) if side == "q" else (None, tab)
+    with pytest.raises(Exception) as e:
+        kernels.qk_rmsnorm_rope(rows, rows, None, eps, q_tab, 1, 64, rows, rows, None, 1e-6, k_tab)
+    assert "unsupported dtype" not in str(e.value)
+    assert eps.alive == [True, True]
+    assert [r() for r in tab.refs] == [None, None]   # and no longer than the call
