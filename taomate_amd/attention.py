@@ -82,10 +82,11 @@ class CausalLTXAttention(nn.Module):
         wp, bp, shape = w.data_ptr(), b.data_ptr(), (n, w.shape[1])
         w_step, b_step = n * w.stride(0) * w.element_size(), n * b.element_size()
         for name in ("to_q", "to_k", "to_v"):
-            lin = self._modules[name]._parameters
-            lw, lb = lin["weight"], lin["bias"]
-            if lw.data_ptr() != wp or lb is None or lb.data_ptr() != bp or lw.shape != shape:
-                self._qkv_packed = None   # a parameter was replaced: drop the stale buffer
+            lin = self._modules.get(name)
+            params = lin._parameters if lin is not None else {}
+            lw, lb = params.get("weight"), params.get("bias")   # absent in a parametrized or wrapped projection
+            if lw is None or lb is None or lw.data_ptr() != wp or lb.data_ptr() != bp or lw.shape != shape:
+                self._qkv_packed = None   # a parameter or projection was replaced: drop the stale buffer
                 return None
             wp += w_step
             bp += b_step

@@ -57,6 +57,50 @@ def test_replacing_a_parameter_ends_the_packing():
     assert m2._packed_qkv() is None
 
 
+class _Adapter(torch.nn.Module):
+    """A projection wrapped the way adapters do: the base's weight and bias as properties."""
+
+    def __init__(self, base):
+        super().__init__()
+        self.base, self.delta = base, torch.nn.Linear(base.in_features, base.out_features, bias=False)
+
+    weight = property(lambda self: self.base.weight)
+    bias = property(lambda self: self.base.bias)
+
+    def forward(self, x):
+        return self.base(x) + self.delta(x)
+
+
+class _BufferLinear(torch.nn.Module):
+    def __init__(self, base):
+        super().__init__()
+        self.register_buffer("weight", base.weight.detach().clone())
+        self.register_buffer("bias", base.bias.detach().clone())
+
+    def forward(self, x):
+        return torch.nn.functional.linear(x, self.weight, self.bias)
+
+
+REPLACED = {
+    "weight_norm": lambda m, n: torch.nn.utils.parametrizations.weight_norm(getattr(m, n)),
+    "adapter": lambda m, n: setattr(m, n, _Adapter(getattr(m, n))),
+    "buffers": lambda m, n: setattr(m, n, _BufferLinear(getattr(m, n))),
+    "no_bias": lambda m, n: setattr(getattr(m, n), "bias", None),
+    "function": lambda m, n: (delattr(m, n), setattr(m, n, torch.nn.functional.normalize)),
+}
+
+
+@pytest.mark.parametrize("name", ["to_q", "to_k", "to_v"])
+@pytest.mark.parametrize("how", list(REPLACED))
+def test_replacing_a_projection_ends_the_packing(how, name):
+    m = _module().fuse_qkv_()
+    REPLACED[how](m, name)
+    assert m._packed_qkv() is None and m._qkv_packed is None
+    x = torch.randn(1, 4, 64)
+    for g_, w_ in zip(_project_qkv(m, x, x), (m.to_q(x), m.to_k(x), m.to_v(x))):
+        assert torch.equal(g_, w_)
+
+
 def test_cross_attention_and_foreign_context_stay_unpacked():
     m = T.CausalLTXAttention(64, context_dim=32, heads=2, dim_head=32).fuse_qkv_()
     assert getattr(m, "_qkv_packed", None) is None
