@@ -35,6 +35,8 @@ from typing import Dict, List, Optional, Tuple
 import torch
 import torch.nn as nn
 import torch.nn.functional as F
+import torch.nn.modules.module as nn_module
+from torch.autograd import forward_ad
 
 from . import kernels
 from .attention import CausalLTXAttention, attention_with_cache, standard_attention_forward
@@ -82,18 +84,39 @@ def timestep_embedding(t: torch.Tensor, dim: int = 256, max_period: int = 10000)
     return torch.cat([torch.cos(emb), torch.sin(emb)], dim=-1)
 
 
+def _is_plain(m: nn.Module, cls: type) -> bool:
+    """Whether calling ``m`` runs ``cls``'s own forward and nothing else: no
+    subclass or parametrization, no forward set on the instance, no compiled
+    call and no forward hooks, its own or global."""
+    return (type(m) is cls and "forward" not in m.__dict__ and m._compiled_call_impl is None
+            and not (m._forward_hooks or m._forward_pre_hooks
+                     or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks))
+
+
+def _is_eager() -> bool:
+    """Whether an op on plain tensors would run as it is written: no gradients,
+    autocast, forward-mode level, function transform, torch function or
+    dispatch mode, trace or compilation sees it."""
+    return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or forward_ad._current_level >= 0
+                or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_function_stack()
+                or torch._C._len_torch_dispatch_stack() or torch.jit.is_tracing() or torch.compiler.is_compiling())
+
+
 def _row_linear(lin: nn.Module, x: torch.Tensor, act: Optional[nn.Module] = None) -> torch.Tensor:
     """``lin(act(x))`` for a few rows (one per sample or frame): a plain bf16
-    nn.Linear without hooks reads its weight once (ltx_skinny_linear); anything
-    else runs as modules."""
-    if (type(lin) is nn.Linear and x.is_cuda and x.dtype == torch.bfloat16 and lin.weight.dtype == torch.bfloat16
-            and not torch.is_grad_enabled() and x.dim() == 2 and 1 <= x.shape[0] <= kernels.SKINNY_MAX_ROWS
-            and x.shape[1] <= kernels.SKINNY_MAX_K and x.shape[1] % 8 == 0
-            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
-            and lin.weight.is_contiguous() and lin.weight.data_ptr() % 16 == 0 and lin.weight.device == x.device
-            and not (lin._forward_hooks or lin._forward_pre_hooks)
-            and (act is None or (type(act) is nn.SiLU and not (act._forward_hooks or act._forward_pre_hooks)))):
-        return kernels.skinny_linear(x, lin.weight, lin.bias, silu=act is not None)
+    nn.Linear in plain eager mode reads its weight once (ltx_skinny_linear);
+    anything else runs as modules."""
+    if (x.is_cuda and _is_plain(lin, nn.Linear) and (act is None or _is_plain(act, nn.SiLU) and not act.inplace)
+            and _is_eager()):
+        w, b = lin.weight, lin.bias
+        if (type(x) is torch.Tensor and x.dtype == torch.bfloat16 and x.dim() == 2
+                and 1 <= x.shape[0] <= kernels.SKINNY_MAX_ROWS and x.shape[1] <= kernels.SKINNY_MAX_K
+                and x.shape[1] % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
+                and all(t is None or type(t) in (nn.Parameter, torch.Tensor) and t.dtype == x.dtype
+                        and t.device == x.device and t.is_contiguous() for t in (w, b))
+                and w.dim() == 2 and w.shape[1] == x.shape[1] and w.data_ptr() % 16 == 0
+                and (b is None or b.shape == w.shape[:1])):
+            return kernels.skinny_linear(x, w, b, silu=act is not None)
     return lin(x if act is None else act(x))
 
 

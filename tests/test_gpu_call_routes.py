@@ -2,6 +2,7 @@
 reference: plain caches in strides and alignments that are attended in place
 or concatenated, key-range splits of partly filled grids, norm rows without
 RoPE tables, and the timestep MLPs with and without the row kernel."""
+import contextlib
 import math
 
 import pytest
@@ -152,3 +153,46 @@ def test_timestep_mlp_routes(dev, rows):
         m(t, torch.bfloat16)
     h.remove()
     assert seen == [1]
+
+
+def _forward_override(m):
+    base = m.linear.forward
+    m.linear.forward = lambda x: base(x) + 1
+
+
+def _strided_bias(m):
+    m.linear.bias = torch.nn.Parameter(torch.stack([m.linear.bias.detach()] * 2, 1)[:, 0])
+
+
+@pytest.mark.parametrize("how", ["forward", "strided_bias", "global_hook", "autocast", "tangent"])
+def test_timestep_mlp_keeps_what_modules_do(dev, how):
+    """What a linear's own call would see or do holds without grad too: a
+    replaced forward, a strided bias, a global hook, autocast to fp16 and a
+    forward-mode tangent give the module path's result bit for bit."""
+    fw = torch.autograd.forward_ad
+    m = dit.AdaLayerNormSingle(512, 6).to(dev, torch.bfloat16)
+    g = gen(7)
+    with torch.no_grad():
+        for p in m.parameters():
+            p.copy_((torch.randn(p.shape, generator=g) * 0.05).to(dev))
+        {"forward": _forward_override, "strided_bias": _strided_bias}.get(how, lambda m: None)(m)
+    x = randn((2, 512), g, torch.bfloat16).to(dev)
+    seen = []
+    hook = torch.nn.modules.module.register_module_forward_hook(lambda *_: seen.append(1)) if how == "global_hook" else None
+    try:
+        with torch.autocast("cuda", torch.float16, enabled=how == "autocast"), \
+                fw.dual_level() if how == "tangent" else contextlib.nullcontext():
+            xin = fw.make_dual(x, torch.ones_like(x)) if how == "tangent" else x
+            with torch.no_grad():
+                out = dit._row_linear(m.linear, xin, m.silu)
+                calls = len(seen)
+                want = m.linear(m.silu(xin))
+            if how == "tangent":
+                (out, t), (want, wt) = fw.unpack_dual(out), fw.unpack_dual(want)
+                assert torch.equal(t, wt)
+    finally:
+        if hook is not None:
+            hook.remove()
+    torch.cuda.synchronize()
+    assert out.dtype == want.dtype and torch.equal(out, want)
+    assert calls == (2 if how == "global_hook" else 0)
