@@ -114,14 +114,25 @@ template <typename T = float>
 T* ptr_as(Opt t) { return static_cast<T*>(ptr(t)); }
 void* stream_of(const at::Tensor& t) { return c10::hip::getCurrentHIPStream(t.device().index()).stream(); }
 
-// Runs an entry point with the GIL released, as ctypes does.
+struct GilReleased {
+  PyThreadState* state = PyEval_SaveThread();
+  ~GilReleased() { PyEval_RestoreThread(state); }
+};
+// Runs enqueue(), which calls the entry point `name`, with the GIL released, as ctypes does.
+template <typename Enqueue>
+void released(const char* name, Enqueue enqueue) {
+  if (api.last_error == nullptr) throw Refused{PyExc_RuntimeError, "the native library is not bound"};
+  int rc;
+  {
+    GilReleased r;
+    rc = enqueue();
+  }
+  if (rc != 0)
+    throw Refused{native_call_error, std::string(name) + " failed (" + std::to_string(rc) + "): " + api.last_error()};
+}
 template <typename Fn, typename... Args>
 void call(const char* name, Fn fn, Args... args) {
-  if (fn == nullptr) throw Refused{PyExc_RuntimeError, "the native library is not bound"};
-  int rc;
-  Py_BEGIN_ALLOW_THREADS rc = fn(args...);
-  Py_END_ALLOW_THREADS if (rc != 0) throw Refused{
-      native_call_error, std::string(name) + " failed (" + std::to_string(rc) + "): " + api.last_error()};
+  released(name, [&] { return fn(args...); });
 }
 
 // ---------------------------------------------------------------- norm + RoPE
@@ -280,18 +291,23 @@ void kv_append_fp8_pair(PyObject* const* a) {
 }
 
 // ------------------------------------------------------------------ attention
-// The split's workspace: one tensor per (device, stream), so that overlapping
-// launches never share one, grown on demand and at most the library's largest
-// plan (24 MiB).  Kept for the life of the process (never destroyed: the
-// allocator may be gone by then).
-at::Tensor workspace(const at::Tensor& q, int64_t need) {
+// The split's workspace: one tensor per (device, stream), grown on demand and
+// at most the library's largest plan.  A call enqueues the attention and the
+// merge of its partials as separate launches, so it holds the workspace's lock
+// until both are in the stream: threads that share a stream (PyTorch's all start
+// on one) take turns.  The lock is taken with the GIL released and given back
+// before the GIL is taken again, so neither waits for the other.  The map is
+// kept for the life of the process (never destroyed: the allocator may be gone
+// by then), and its entries never move.
+struct Workspace {
+  std::mutex mu;
+  at::Tensor buf;
+};
+Workspace& workspace(const at::Tensor& q, void* stream) {
   static std::mutex mu;
-  static auto* kept = new std::map<std::pair<int, void*>, at::Tensor>;
-  const std::pair<int, void*> key{q.device().index(), stream_of(q)};
+  static auto* kept = new std::map<std::pair<int, void*>, Workspace>;
   std::lock_guard<std::mutex> lock(mu);
-  at::Tensor& ws = (*kept)[key];
-  if (!ws.defined() || ws.numel() < need) ws = at::empty({need}, q.options().dtype(at::kByte));
-  return ws;
+  return (*kept)[{q.device().index(), stream}];
 }
 
 PyObject *str_k, *str_v, *str_ks, *str_vs;
@@ -404,34 +420,35 @@ void flash_attn(PyObject* const* a) {
       value_error("flash_attn: key_lens must hold " + std::to_string(B) + " counts in [0, " + std::to_string(lk) + "]");
   }
   void* st = stream_of(q);
-  at::Tensor ws;
-  int64_t ws_bytes = 0;
-  if (!noalloc) {
-    int64_t need = 0;
-    call("ltx_flash_attn_workspace_size", api.flash_attn_workspace_size, B, Lq, H, D, &need);
-    if (need > 0) {
-      ws = workspace(q, need);
-      ws_bytes = ws.numel();
-    }
-  }
-  void* wsp = ws.defined() ? ws.data_ptr() : nullptr;
-  if (own_bs) {
-    call("ltx_flash_attn_fwd_plain", api.flash_attn_fwd_plain, ptr(&q), B, Lq, H, D, q.stride(0), q.stride(1),
-         q.stride(2), (int64_t)n, kp, vp, lens, seg_bs, k0.stride(1), k0.stride(2), ptr(&out), out.stride(0),
-         out.stride(1), out.stride(2), ptr_as(lse), scale, wsp, ws_bytes, st);
+  const int64_t* kl_data = a[8] != Py_None ? kl.data() : nullptr;
+  auto general = [&](auto fn, auto... tail) {
+    return fn(ptr(&q), B, Lq, H, D, q.stride(0), q.stride(1), q.stride(2), (int64_t)n, kp, vp, lens, k0.stride(0),
+              k0.stride(1), k0.stride(2), v0.stride(0), v0.stride(1), v0.stride(2), v0.stride(3), kv_code,
+              fp8 ? ksp : nullptr, fp8 ? vsp : nullptr, sc_bs, sc_hs, frame, ptr_as(mask), mask_bs, kl_data, ptr(&out),
+              out.stride(0), out.stride(1), out.stride(2), ptr_as(lse), scale, tail...);
+  };
+  if (noalloc) {
+    released("ltx_flash_attn_fwd_noalloc", [&] { return general(api.flash_attn_fwd_noalloc, st); });
     return;
   }
-  auto run = [&](const char* name, auto fn, auto... tail) {
-    call(name, fn, ptr(&q), B, Lq, H, D, q.stride(0), q.stride(1), q.stride(2), (int64_t)n, kp, vp, lens,
-         k0.stride(0), k0.stride(1), k0.stride(2), v0.stride(0), v0.stride(1), v0.stride(2), v0.stride(3), kv_code,
-         fp8 ? ksp : nullptr, fp8 ? vsp : nullptr, sc_bs, sc_hs, frame, ptr_as(mask), mask_bs,
-         a[8] != Py_None ? kl.data() : nullptr, ptr(&out), out.stride(0), out.stride(1), out.stride(2), ptr_as(lse),
-         scale, tail...);
-  };
-  if (noalloc)
-    run("ltx_flash_attn_fwd_noalloc", api.flash_attn_fwd_noalloc, st);
-  else
-    run("ltx_flash_attn_fwd", api.flash_attn_fwd, wsp, ws_bytes, st);
+  int64_t need = 0;
+  call("ltx_flash_attn_workspace_size", api.flash_attn_workspace_size, B, Lq, H, D, &need);
+  released(own_bs ? "ltx_flash_attn_fwd_plain" : "ltx_flash_attn_fwd", [&] {
+    std::unique_lock<std::mutex> lock;
+    void* wsp = nullptr;
+    int64_t ws_bytes = 0;
+    if (need > 0) {
+      Workspace& ws = workspace(q, st);
+      lock = std::unique_lock<std::mutex>(ws.mu);
+      if (!ws.buf.defined() || ws.buf.numel() < need) ws.buf = at::empty({need}, q.options().dtype(at::kByte));
+      wsp = ws.buf.data_ptr();
+      ws_bytes = ws.buf.numel();
+    }
+    if (!own_bs) return general(api.flash_attn_fwd, wsp, ws_bytes, st);
+    return api.flash_attn_fwd_plain(ptr(&q), B, Lq, H, D, q.stride(0), q.stride(1), q.stride(2), (int64_t)n, kp, vp,
+                                    lens, seg_bs, k0.stride(1), k0.stride(2), ptr(&out), out.stride(0),
+                                    out.stride(1), out.stride(2), ptr_as(lse), scale, wsp, ws_bytes, st);
+  });
 }
 
 // ---------------------------------------------------------------------- AdaLN
