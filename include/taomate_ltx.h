@@ -280,7 +280,7 @@ int ltx_flash_attn_fwd_plain(const void* q, int64_t B, int64_t Lq, int64_t H, in
  *   one device share the array and race: serialise them (one stream, or
  *   events).
  */
-#define LTX_NOALLOC_SCRATCH_BYTES (24ll << 20)
+#define LTX_NOALLOC_SCRATCH_BYTES (25ll << 20)
 int ltx_flash_attn_fwd_noalloc(const void* q, int64_t B, int64_t Lq, int64_t H, int64_t D,
                                int64_t q_bs, int64_t q_ls, int64_t q_hs, int64_t n_segments,
                                const void* const* k_ptrs, const void* const* v_ptrs,

@@ -17,7 +17,7 @@ LIB_NAME = "libtaomate_ltx.so"
 F32, BF16, F8E4M3 = 0, 1, 2
 MAX_SEGMENTS = 16
 MAX_KEYLEN_BATCH = 16  # LTX_MAX_KEYLEN_BATCH
-NOALLOC_SCRATCH_BYTES = 24 << 20  # LTX_NOALLOC_SCRATCH_BYTES
+NOALLOC_SCRATCH_BYTES = 25 << 20  # LTX_NOALLOC_SCRATCH_BYTES
 ABI_VERSION = 2
 
 _i64 = ctypes.c_int64

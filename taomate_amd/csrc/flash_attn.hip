@@ -78,8 +78,9 @@ struct FlashParams {
   // and 2u + 1, which lie in one (batch, head) and share every K/V tile;
   // n_full and split count units, and the tail q-tiles start at 2 n_full.
   int pair;
-  uint16_t* part_o;  // [tail tiles * split][kBM][D] bf16 O / l of the key range (0 where l = 0)
-  float* part_ml;     // [tail tiles * split][kBM][2] running max (log2) and sum
+  void* part_o;    // [tail tiles * split][kBM][D] O / l of the key range (0 where l = 0), bf16 or
+  int part_f32;    // float32 (see plan_split)
+  float* part_ml;  // [tail tiles * split][kBM][2] running max (log2) and sum
   float scale;       // softmax scale applied to q.k
   float scale_log2;  // scale * log2(e)
 };
@@ -288,7 +289,9 @@ __device__ __forceinline__ WorkItem pair_work(const FlashParams& p, int bid, int
 }
 
 // Epilogue shared by the kernels: normalise and store a whole q-tile, or
-// store a key range's partial result (unnormalised O, running max and sum).  oacc holds O^T fragments (lane: query li,
+// store a key range's partial result (O normalised by its own sum, in bf16 or, with
+// MAYBE_F32 and where the launch plan says so, in float32; running max and
+// sum).  oacc holds O^T fragments (lane: query li,
 // d = db*32 + 8*(r/4) + 4*hg + r%4); m_run / l_tot are per query.
 //
 // stage (the pipelined kernels): this wave's 32 x (D + 8) bf16 region of LDS,
@@ -302,13 +305,26 @@ __device__ __forceinline__ WorkItem pair_work(const FlashParams& p, int bid, int
 // after it 1.5 us faster.  Every wave of the workgroup calls it (two
 // barriers inside), with one path for the whole workgroup (a whole q-tile or
 // a key range, and o_al16).
-template <int D>
+template <int D, bool MAYBE_F32>
 __device__ __forceinline__ void finish_tile(const FlashParams& p, const WorkItem& w, int b, int h,
                                             int qt, int row, const f32x16_t (&oacc)[D / 32], float m_run,
                                             float l_tot, uint16_t* stage = nullptr) {
   constexpr int DB = D / 32;
   const int hg = (threadIdx.x & 63) >> 5;  // row: this lane's query inside the q-tile
   const int qi = qt * kBM + row;
+  if (MAYBE_F32 && w.piece >= 0 && p.part_f32) {
+    const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
+    float* po = static_cast<float*>(p.part_o) + ((int64_t)w.piece * kBM + row) * D + 4 * hg;
+#pragma unroll
+    for (int d = 0; d < DB; ++d)
+#pragma unroll
+      for (int g4 = 0; g4 < 4; ++g4)
+        *reinterpret_cast<float4*>(po + d * 32 + 8 * g4) =
+            make_float4(oacc[d][4 * g4] * inv, oacc[d][4 * g4 + 1] * inv, oacc[d][4 * g4 + 2] * inv,
+                        oacc[d][4 * g4 + 3] * inv);
+    if (hg == 0) *reinterpret_cast<float2*>(p.part_ml + ((int64_t)w.piece * kBM + row) * 2) = make_float2(m_run, l_tot);
+    return;
+  }
   if (stage != nullptr && (w.piece >= 0 || p.o_al16)) {
     constexpr int RS = D + 8;   // staging row stride (elements)
     constexpr int CPR = D / 8;  // 16-byte chunks per row
@@ -338,7 +354,7 @@ __device__ __forceinline__ void finish_tile(const FlashParams& p, const WorkItem
       if (p.lse != nullptr && hg == 0 && qi < p.Lq)
         p.lse[((int64_t)b * p.H + h) * p.Lq + qi] = (m_run + __log2f(l_tot)) / kLog2e;
     } else {
-      uint16_t* po = p.part_o + ((int64_t)w.piece * kBM + row0) * D;
+      uint16_t* po = static_cast<uint16_t*>(p.part_o) + ((int64_t)w.piece * kBM + row0) * D;
 #pragma unroll
       for (int i = 0; i < D / 16; ++i) {
         const int c = i * 64 + lane, r = c / CPR, cc = c % CPR;
@@ -368,9 +384,9 @@ __device__ __forceinline__ void finish_tile(const FlashParams& p, const WorkItem
   }
   // ---- partial result of one key range: combined by flash_combine_kernel.
   // O is stored normalised by the range's own sum and rounded to bf16 (the
-  // output's precision), so the partials cost a quarter of fp32 O traffic;
-  // the combine weighs each range by its sum and maximum. ----
-  uint16_t* po = p.part_o + ((int64_t)w.piece * kBM + row) * D;
+  // output's precision), half the bytes of float32; the combine weighs each
+  // range by its sum and maximum. ----
+  uint16_t* po = static_cast<uint16_t*>(p.part_o) + ((int64_t)w.piece * kBM + row) * D;
   const float inv = l_tot > 0.0f ? 1.0f / l_tot : 0.0f;
 #pragma unroll
   for (int d = 0; d < DB; ++d)
@@ -385,8 +401,7 @@ __device__ __forceinline__ void finish_tile(const FlashParams& p, const WorkItem
 }
 
 // Epilogue of the pipelined kernels: normalise and store a wave's 32 rows of
-// a whole q-tile, or store a key range's partial result (O normalised by its
-// own sum, running max and sum).  oacc[d][n] holds O^T fragments (lane: query
+// a whole q-tile, or store a key range's partial result (as finish_tile).  oacc[d][n] holds O^T fragments (lane: query
 // row0 + 16 n + li, channels 16 d + 4 lg + r); m_run / l_tot are per query.
 //
 // stage: this wave's 32 x D bf16 region of LDS, free once every wave is past
@@ -399,8 +414,9 @@ __device__ __forceinline__ void finish_tile(const FlashParams& p, const WorkItem
 // 152.6 us with streaming stores at the 1152 x 4608 chunk, and the launch
 // after it 1.5 us faster.  Every wave of the workgroup calls it (two
 // barriers inside), with one path for the whole workgroup (a whole q-tile or
-// a key range, and o_al16).
-template <int D>
+// a key range, part_f32 and o_al16).  Float32 partials go straight from the
+// accumulators, 16 bytes per lane.
+template <int D, bool MAYBE_F32>
 __device__ __forceinline__ void finish_rows(const FlashParams& p, const WorkItem& w, int b, int h, int qt, int row0,
                                             const f32x4_t (&oacc)[D / 16][2], const float (&m_run)[2],
                                             const float (&l_tot)[2], uint16_t* stage) {
@@ -411,7 +427,14 @@ __device__ __forceinline__ void finish_rows(const FlashParams& p, const WorkItem
     return make_uint2(pack_bf16x2(oacc[d][n][0] * inv[n], oacc[d][n][1] * inv[n]),
                       pack_bf16x2(oacc[d][n][2] * inv[n], oacc[d][n][3] * inv[n]));
   };
-  if (w.piece < 0 && !p.o_al16) {  // output rows that are only 8-byte aligned
+  if (MAYBE_F32 && w.piece >= 0 && p.part_f32) {
+#pragma unroll
+    for (int n = 0; n < 2; ++n) {
+      float* po = static_cast<float*>(p.part_o) + ((int64_t)w.piece * kBM + row0 + 16 * n + li) * D + 4 * lg;
+#pragma unroll
+      for (int d = 0; d < D / 16; ++d) *reinterpret_cast<f32x4_t*>(po + d * 16) = oacc[d][n] * inv[n];
+    }
+  } else if (w.piece < 0 && !p.o_al16) {  // output rows that are only 8-byte aligned
 #pragma unroll
     for (int n = 0; n < 2; ++n) {
       const int qi = qt * kBM + row0 + 16 * n + li;
@@ -430,7 +453,7 @@ __device__ __forceinline__ void finish_rows(const FlashParams& p, const WorkItem
                                   (lg & 1) * 4) = packed(d, n);
     __syncthreads();
     const int64_t obase = b * p.o_bs + h * p.o_hs;
-    uint16_t* po = w.piece < 0 ? nullptr : p.part_o + ((int64_t)w.piece * kBM + row0) * D;
+    uint16_t* po = w.piece < 0 ? nullptr : static_cast<uint16_t*>(p.part_o) + ((int64_t)w.piece * kBM + row0) * D;
 #pragma unroll
     for (int i = 0; i < D / 16; ++i) {
       const int c = i * 64 + lane, r = c / CPR, cc = c % CPR;
@@ -457,16 +480,16 @@ constexpr int kMaxSplit = 8;  // key ranges a tail q-tile may be cut into
 
 // Combines the `split` partial results of every tail q-tile, launched after the
 // attention kernel on the same stream: out = sum_i w_i o_i / sum_i w_i with
-// w_i = l_i 2^(m_i - max m) and o_i the range's normalised output.  One thread
-// per (query row, 8 output columns): every piece's (max, sum) and 16-byte O
-// chunk are loaded up front, so each thread waits for one round of loads.
+// w_i = l_i 2^(m_i - max m) and o_i the range's normalised output (F32: in
+// float32).  One thread per (query row, 8 output columns): every piece's (max,
+// sum) and 16- or 32-byte O chunk are loaded up front, so each thread waits for one round of loads.
 // The output is written as two 8-byte halves (the entry point guarantees
 // 8-byte aligned output rows); the workspace partials are 16-byte aligned.
 constexpr int kCombineCols = 8;
 template <int D>
 constexpr int combine_wg_per_tile() { return kBM / (256 / (D / kCombineCols)); }
 
-template <int D>
+template <int D, bool F32>
 __global__ void __launch_bounds__(256) flash_combine_kernel(const FlashParams p) {
   constexpr int CG = D / kCombineCols;  // 8-column groups per row
   constexpr int ROWS = 256 / CG;        // rows per workgroup
@@ -483,12 +506,16 @@ __global__ void __launch_bounds__(256) flash_combine_kernel(const FlashParams p)
   if (q >= p.Lq) return;
   const int64_t first = (int64_t)tail * p.split;
   f32x2_t ml[kMaxSplit];
-  uint4 o[kMaxSplit];
+  typedef std::conditional_t<F32, float, uint16_t> part_t;
+  constexpr int CW = kCombineCols * sizeof(part_t) / 16;  // 16-byte words of a chunk
+  uint4 o[kMaxSplit][CW];
 #pragma unroll
   for (int i = 0; i < kMaxSplit; ++i) {
     if (i < p.split) {
       ml[i] = *reinterpret_cast<const f32x2_t*>(p.part_ml + ((first + i) * kBM + r) * 2);
-      o[i] = *reinterpret_cast<const uint4*>(p.part_o + ((first + i) * kBM + r) * D + cg * kCombineCols);
+      const part_t* po = static_cast<const part_t*>(p.part_o) + ((first + i) * kBM + r) * D + cg * kCombineCols;
+#pragma unroll
+      for (int c = 0; c < CW; ++c) o[i][c] = reinterpret_cast<const uint4*>(po)[c];
     }
   }
   float mmax = -INFINITY;
@@ -502,11 +529,18 @@ __global__ void __launch_bounds__(256) flash_combine_kernel(const FlashParams p)
     if (i < p.split) {
       const float wgt = ml[i][0] == -INFINITY ? 0.0f : __builtin_amdgcn_exp2f(ml[i][0] - mmax) * ml[i][1];
       lsum += wgt;
-      const uint32_t w[4] = {o[i].x, o[i].y, o[i].z, o[i].w};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        acc[2 * e] += wgt * bf16_bits_to_f32(w[e] & 0xFFFFu);
-        acc[2 * e + 1] += wgt * bf16_bits_to_f32(w[e] >> 16);
+      for (int c = 0; c < CW; ++c) {
+        const uint32_t w[4] = {o[i][c].x, o[i][c].y, o[i][c].z, o[i][c].w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          if constexpr (F32) {
+            acc[4 * c + e] += wgt * __uint_as_float(w[e]);
+          } else {
+            acc[2 * e] += wgt * bf16_bits_to_f32(w[e] & 0xFFFFu);
+            acc[2 * e + 1] += wgt * bf16_bits_to_f32(w[e] >> 16);
+          }
+        }
       }
     }
   }
@@ -756,7 +790,7 @@ __global__ void __launch_bounds__(256, 2) flash_fwd_masked_kernel(const FlashPar
   }
 
   // ---- epilogue: combine the two lane halves' sums, then store or publish ----
-  finish_tile<D>(p, wi, b, h, qt, (int)(threadIdx.x >> 6) * 32 + (int)(threadIdx.x & 31), oacc, m_run,
+  finish_tile<D, false>(p, wi, b, h, qt, (int)(threadIdx.x >> 6) * 32 + (int)(threadIdx.x & 31), oacc, m_run,
                  pair_sum(l_run));
 }
 
@@ -1347,7 +1381,7 @@ __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
   static_assert((PAIR ? 8 : 4) * 32 * D <= 2 * (KBUF + VBUF), "output staging region");
   const int owave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const float l_tot[2] = {quad_sum(l_run[0]), quad_sum(l_run[1])};
-  finish_rows<D>(p, wi, b, h, qt, wave * 32, oacc, m_run, l_tot, smem + owave * 32 * D);
+  finish_rows<D, !PAIR || (VTOK && D == 64)>(p, wi, b, h, qt, wave * 32, oacc, m_run, l_tot, smem + owave * 32 * D);
 }
 
 // The 32x32x16 body: the fp8 kernels, and bf16 key-major V where the part is
@@ -1912,7 +1946,7 @@ __device__ __forceinline__ void flash_mfma32_body(const FlashParams& p) {
   static_assert(4 * 32 * (D + 8) <= 2 * KBUF && 4 * 32 * (D + 8) <= 2 * VBUF, "output staging region");
   const int owave = PAIR ? wave : (int)(threadIdx.x >> 6);
   uint16_t* stage = (PAIR && grp == 1 ? &vbuf[0][0] : &kbuf[0][0]) + owave * 32 * (D + 8);
-  finish_tile<D>(p, wi, b, h, qt, owave * 32 + (int)(threadIdx.x & 31), oacc, m_run, pair_sum(l_run), stage);
+  finish_tile<D, !PAIR>(p, wi, b, h, qt, owave * 32 + (int)(threadIdx.x & 31), oacc, m_run, pair_sum(l_run), stage);
 }
 
 // KV operands of a kernel instance: bf16 with key-major V (kKeyMajorV32: on
@@ -1947,7 +1981,11 @@ int launch_combine(const FlashParams& p, hipStream_t st) {
   if (p.split <= 1) return LTX_OK;
   const int64_t tail = (int64_t)p.B * p.H * p.n_qtiles - (p.pair ? 2 * (int64_t)p.n_full : p.n_full);
   const int64_t wg_per_tile = combine_wg_per_tile<D>();
-  hipLaunchKernelGGL((flash_combine_kernel<D>), dim3((unsigned)(tail * wg_per_tile)), dim3(256), 0, st, p);
+  const dim3 grid((unsigned)(tail * wg_per_tile));
+  if (p.part_f32)
+    hipLaunchKernelGGL((flash_combine_kernel<D, true>), grid, dim3(256), 0, st, p);
+  else
+    hipLaunchKernelGGL((flash_combine_kernel<D, false>), grid, dim3(256), 0, st, p);
   LTX_LAUNCH_CHECK("ltx_flash_attn_fwd (combine)");
   return LTX_OK;
 }
@@ -1993,8 +2031,8 @@ using namespace ltx;
 // the template has its own).
 constexpr int kMaxDevices = 64;
 struct Slots {
-  int slots;   // resident workgroups (0: unknown, no split is planned)
-  int pieces;  // key-range pieces a split tail aims for (see plan_split)
+  int slots;  // resident workgroups (0: unknown, no split is planned)
+  int cus;
 };
 template <auto Kernel>
 Slots resident_slots(int threads = 256) {
@@ -2010,117 +2048,10 @@ Slots resident_slots(int threads = 256) {
       return;
     }
     occ = occ > 0 ? occ : 1;
-    slots[dev] = Slots{cus * occ, cus};  // pieces: one per CU until flash_slots says otherwise
+    slots[dev] = Slots{cus * occ, cus};
   });
   return slots[dev];
 }
-
-// Tail q-tiles (those past the last whole round of resident slots) and how
-// many key ranges each is cut into: about s.pieces pieces in all.  For the
-// bf16 pipelined kernel that is one per CU.  Of the workgroups one CU holds,
-// the oldest one's waves win the issue arbitration: with two of its 4-wave
-// workgroups per CU the older finishes its q-tile about a quarter before the
-// younger, so one slot per CU frees early.  Pieces that fill just those
-// slots run beside the younger workgroups' last stretch; pieces for every
-// slot (twice as many, half as long) leave their second half to start only
-// when the younger workgroups end, with a CU half busy until they drain
-// (193.7 against 184.8 us for the bf16 step at 1152 x 4608, 8 against 4
-// pieces per tail q-tile).  The fp8 kernel measured the other way round
-// (194-196 against 200-202 us) while its per-tile barrier also waited for
-// the register-staged loads; without that wait it gains from one piece per
-// CU too (187.6 against 180.4 us).  The staged kernel's pieces fill every
-// slot.  Each piece keeps >= 4 key tiles behind a whole round.  A grid
-// that is a single partial round (fewer q-tiles than slots: the 75-query
-// audio and V2A calls, 64 q-tiles at B = 2 and 32 heads) is split too, into
-// pieces of >= 2 key tiles, so its few workgroups spread over the CUs: V2A
-// 75 x 1152 16.0 -> 12.5 us, audio self-attention 75 x 675 14.2 -> 12.6 us.
-// Zero tail tiles: no split.
-//
-// The kernels that hold two workgroups per CU choose the split by split_cost:
-// with one piece per CU as the only rule, tails of more than half the CUs ran
-// whole.  Measured at 32 heads x 128, B = 2, bf16: 3 q-tiles per head (192
-// workgroups) over 10368 keys 191 us whole, 146 in two ranges; 5 per head
-// 252 and 225; 13 per head (a tail of 320) 518 and 486; over 4608 keys 84 and
-// 69, 113 and 109, 235 and 226; over 2048 keys and fewer whole is as fast and
-// stays.  The search starts at one piece per CU and only goes finer: fewer,
-// longer pieces average out less of their bf16 partials' rounding.  With the
-// count free, 98 of 264 grids of 75 to 300 queries over 330 to 2600 keys had a
-// larger error against float64 than one piece per CU gives (by up to 1.9 %),
-// with this floor none has.  75 x 675 at 32 x 64, B = 1, takes 13.0 -> 11.4 us
-// with it (token-major V); 300 x 330 at 16 x 64, B = 2, is 1.24 times as long
-// as whole.  The pair kernel's rule stays as it is: at 6, 12 and 14 q-tiles per
-// head its partly filled rounds measured no slower than any split (the CUs
-// that work run faster while others idle; the part is power bound).
-inline int64_t workspace_bytes_for(int64_t tail, int64_t split, int64_t D) {
-  return tail * split * kBM * (2 * 4 + D * 2);  // (max, sum) fp32 + bf16 O row
-}
-
-// No plan's partials exceed the no-allocation entry point's scratch array, so
-// both entry points plan alike.
-inline int split_limit(int64_t tail_qtiles, int64_t D) {
-  const int64_t n = LTX_NOALLOC_SCRATCH_BYTES / workspace_bytes_for(tail_qtiles, 1, D);
-  return (int)(n < kMaxSplit ? n : kMaxSplit);
-}
-
-// Time of `tail` q-tiles of `ntiles` key tiles in `sp` ranges each, in units
-// of a key tile's time with two workgroups on every CU.  A round of r
-// workgroups of t tiles takes t when every slot is filled, 0.75 t + a share
-// for the CUs with two when r is more than one per CU, and 0.57 t with one
-// per CU (0.43 t behind whole rounds, whose older workgroups end early and
-// free their slots); 2 per round for the pieces' prologue and epilogue, and
-// 2.5 + 0.002 per piece for the combine kernel (half as much again at D = 64,
-// whose tiles are shorter).
-inline float split_cost(int64_t tail, int sp, int ntiles, Slots s, bool after_full, int64_t D) {
-  const int64_t m = tail * sp, whole = m / s.slots, rem = m % s.slots;
-  const float t = (float)((ntiles + sp - 1) / sp), k = D == 64 ? 1.5f : 1.0f;
-  float c = (float)whole * (t + 2.0f * k);
-  if (rem > s.pieces)
-    c += t * (0.75f + 0.25f * (float)(rem - s.pieces) / (float)s.pieces) + 2.0f * k;
-  else if (rem > 0)
-    c += t * (after_full || whole > 0 ? 0.43f : 0.57f) + 2.0f * k;
-  return sp > 1 ? c + k * (2.5f + 0.002f * (float)m) : c;
-}
-
-inline void plan_split(int64_t nq, int ntiles, Slots s, int64_t D, int per_unit, int64_t* n_full, int* split) {
-  *n_full = nq;
-  *split = 1;
-  const int slots = s.slots;
-  if (slots <= 0 || nq % slots == 0) return;
-  const int64_t full = (nq / slots) * slots;
-  const int64_t tail = nq - full;
-  // pieces keep >= 4 key tiles behind a whole round, >= 2 when the grid is
-  // a single partial round (its few workgroups would leave most CUs idle)
-  const int min_tiles = full > 0 ? 4 : 2;
-  int most = split_limit(tail * per_unit, D);
-  if (most > ntiles / min_tiles) most = ntiles / min_tiles;
-  int sp = (int)(s.pieces / tail);
-  sp = sp > most ? most : sp;
-  sp = sp < 1 ? 1 : sp;
-  if (slots == 2 * s.pieces) {
-    float best = split_cost(tail, sp, ntiles, s, full > 0, D);
-    for (int i = sp + 1; i <= most; ++i) {
-      const float c = split_cost(tail, i, ntiles, s, full > 0, D);
-      if (c < 0.94f * best) {
-        best = c;
-        sp = i;
-      }
-    }
-  }
-  if (sp < 2) return;
-  *n_full = full;
-  *split = sp;
-}
-
-// Partial bytes that plan_split may ask for, whatever the key count.
-inline int64_t split_bytes_bound(int64_t nq, Slots s, int64_t D, int per_unit) {
-  if (s.slots <= 0 || nq % s.slots == 0) return 0;
-  const int64_t tail = (nq % s.slots);
-  int64_t sp = split_limit(tail * per_unit, D);
-  if (s.slots != 2 * s.pieces && sp > s.pieces / tail) sp = s.pieces / tail;
-  return sp > 1 ? workspace_bytes_for(tail * per_unit, sp, D) : 0;
-}
-
-inline int64_t round256(int64_t x) { return (x + 255) / 256 * 256; }
 
 // The kernel family a call takes: the masked staged kernel for a key mask,
 // else the pipelined one of its KV kind (the pair instance when the q-tiles
@@ -2139,28 +2070,129 @@ Slots slots_for(FlashPath path, bool pair) {
     case kPathFp8:
       return pair ? resident_slots<flash_fwd_pair_kernel<D, kFp8>>(512)
                   : resident_slots<flash_fwd_pipe_kernel<D, kFp8>>();
-    default: {
-      // pieces: one per slot for the staged kernel, one per CU for the others (plan_split)
-      Slots s = resident_slots<flash_fwd_masked_kernel<D>>();
-      s.pieces = s.slots;
-      return s;
-    }
+    default:
+      return resident_slots<flash_fwd_masked_kernel<D>>();
   }
 }
 inline Slots flash_slots(int64_t D, FlashPath path, bool pair) {
   return D == 128 ? slots_for<128>(path, pair) : slots_for<64>(path, pair);
 }
 
+struct Split {
+  int64_t n_full;  // work units that run whole
+  int n;           // key ranges of each of the others
+  bool f32;        // the ranges' partial O in float32
+  // partial rows of `units` work units of `per_unit` q-tiles, and their bytes:
+  // (max, sum) in float32 for every row, then the O rows
+  int64_t rows(int64_t units, int per_unit) const { return n > 1 ? (units - n_full) * per_unit * n * kBM : 0; }
+  int64_t bytes(int64_t units, int per_unit, int64_t D) const {
+    return rows(units, per_unit) * (2 * 4 + D * (f32 ? 4 : 2));
+  }
+};
+
+// Which work units (q-tiles, or the pair kernel's units of two) are cut into
+// key ranges, and into how many.  Whole rounds of resident workgroups run whole;
+// the rest, the tail, is cut so that its workgroups spread over the CUs.  Pieces
+// keep >= 4 key tiles behind a whole round, >= 2 in a grid that is a single
+// partial round (the 75-query audio and V2A calls: V2A 75 x 1152 16.0 -> 12.5
+// us, audio self-attention 75 x 675 14.2 -> 12.6 us).
+//
+// Base: one piece per CU.  Of the workgroups one CU holds, the oldest one's
+// waves win the issue arbitration: with two 4-wave workgroups per CU the older
+// finishes its q-tile about a quarter before the younger, so one slot per CU
+// frees early.  Pieces that fill just those slots run beside the younger
+// workgroups' last stretch; pieces for every slot leave their second half to
+// start only when the younger workgroups end (1152 x 4608 bf16: 193.7 against
+// 184.8 us for the step with 8 against 4 pieces per tail q-tile; fp8 187.6
+// against 180.4 us).  The masked kernel's pieces fill every slot.  The pair
+// kernel keeps to the base: at 6, 12 and 14 q-tiles per head its partly filled
+// rounds measured no slower than any split.
+//
+// What may be split further is bounded by exactness.  A range's O is rounded to
+// bf16 before the merge, which makes the error against float64 1.22 times the
+// whole call's where all rows are split; over more ranges it averages out a
+// little.  So units that the base leaves whole (a tail of more than half the
+// CUs) keep their float32 sums: they are split only with float32 partials
+// (0.96 to 1.003 times the whole call's error), whose traffic (25 MB written and
+// read again for 384 pieces at D = 128) costs 10 to 15 us, and so only over
+// enough keys.  Measured in us, whole against
+// split, by tail and ranges (B * H = 16 to 64 heads; KT key tiles, for fp8 KT
+// tiles in 330-token frames):
+//   up to 1/3 of the slots, 3 ranges: bf16 D = 128 tail 160 at KT 41: 38.6 / 40.2,
+//     54: 48.2 / 45.4, 162: 133 / 103; D = 64 at 41: 30.1 / 28.3, 108: 70.3 / 48.9;
+//     fp8 at 24: 41.4 / 38.6, 84: 125 / 78
+//   up to 1/2, 2 ranges, or 4 where those fill at most 1.5 rounds: tail 192 D = 128
+//     at 72: 64.2 / 68.5, 108: 94.0 / 98.1, 162: 194 / 137; D = 64 at 72: 48.9 / 43.4,
+//     108: 70.9 / 58.1; fp8 at 24: 41.5 / 44.3, 36: 59.1 / 55.7, 84: 127 / 97
+//   up to 2/3, 3 ranges: tail 320 D = 128 at 54: 81.8 / 83.3, 72: 107 / 103, 162: 235 / 211;
+//     fp8 at 36: 79.5 / 81.4, 48: 102 / 97; token-major at 54: 89.2 / 87.1
+//   up to 3/4, 2 ranges: tail 352 D = 128 at 72: 109 / 110, 108: 161 / 155; fp8 at 48:
+//     102 / 105, 84: 171 / 164
+//   above: no split gains (tail 416 and 448: 1.03 to 1.3 times as long up to 6912 keys)
+// More ranges in bf16 than the base cost no exactness: grids of one partial
+// round take one piece per slot where the base gives 2 or 3 ranges (fp8: 4 too)
+// and the keys are long: tail 96, 5 against 2 ranges, D = 128 at 41: 27.6 / 28.0,
+// 72: 36.1 / 39.9; D = 64 at 41: 20.0 / 22.4; fp8 at 24: 26.6 / 29.9, 48: 35.9 / 46.5.
+//
+// Token-major calls came from a staged kernel whose pieces filled every slot,
+// three workgroups per CU at D = 64, and keep at least as many ranges in a
+// partial round (V2A 75 x 1152: error 1.020 times with 4 instead of 8), or take
+// float32 partials where fewer are faster (tail 80 at D = 64, KT 18: 3 ranges in
+// float32 16.0 us, 8 in bf16 19.2), or run whole over few keys (tail 160 D = 128 at
+// 18: 24.4 against 28.9 us in 3 ranges in float32).  Behind whole rounds four bf16 ranges are as exact as
+// eight (1.0005), two or three are not.
+inline Split plan_split(int64_t units, int ntiles, FlashPath path, bool pair, int64_t D) {
+  const Slots s = flash_slots(D, path, pair);
+  if (s.slots <= 0 || units % s.slots == 0) return {units, 1, false};
+  const int64_t S = s.slots, full = units / S * S, tail = units - full;
+  const bool one_round = full == 0, token = path == kPathTokenMajor, fp8 = path == kPathFp8, d64 = D == 64;
+  const bool two_per_cu = !pair && path != kPathMasked && S == 2 * s.cus;
+  auto below = [](int64_t n, int64_t limit) { return n < limit ? n : limit; };
+
+  int64_t n = (path == kPathMasked ? S : s.cus) / tail;
+  bool f32 = false;
+  if (token && one_round) {
+    const int64_t least = d64 ? (S + S / 2) / tail : S / tail;
+    if (!d64 || (two_per_cu && (4 * tail <= s.cus || (3 * tail > S && 2 * tail <= S))))
+      n = least;
+    else if (two_per_cu && ntiles >= (n >= 3 ? 128 : n == 2 ? 48 : 36))
+      n = S / tail;
+    f32 = n < below(least, kMaxSplit);
+    if (two_per_cu && 2 * tail > s.cus && ntiles < (d64 || 3 * tail > S ? 36 : 24)) n = 1;
+    if (f32 && ntiles < (2 * tail < s.cus || two_per_cu ? 16 : 27)) n = 1;
+  } else if (token) {
+    f32 = d64 || n < 4;
+  } else if (two_per_cu && one_round && n >= 2 && n <= (fp8 ? 4 : 3) && ntiles >= (fp8 ? 36 : d64 ? 40 : 72)) {
+    n = S / tail;
+  }
+  if (two_per_cu && n < 2) {
+    f32 = true;
+    if (3 * tail <= S)
+      n = ntiles >= (fp8 ? 24 : d64 ? 40 : 54) ? 3 : 1;
+    else if (2 * tail <= S)
+      n = ntiles < (fp8 ? 36 : d64 ? 72 : 128) ? 1 : 8 * tail <= 3 * S && ntiles >= 54 ? 4 : 2;
+    else if (3 * tail <= 2 * S)
+      n = ntiles >= (fp8 ? 48 : token ? 54 : 72) ? 3 : 1;
+    else if (4 * tail <= 3 * S)
+      n = ntiles >= (fp8 ? 66 : 100) ? 2 : 1;
+  }
+  n = below(below(n, kMaxSplit), ntiles / (one_round ? 2 : 4));
+  return n >= 2 ? Split{full, (int)n, f32} : Split{units, 1, false};
+}
+
+inline int64_t round256(int64_t x) { return (x + 255) / 256 * 256; }
+
 // Key-major bf16 calls that keep the 32x32x16 kernel: the 4-wave kernel with
-// little more than one workgroup per CU, or fewer than 16 key tiles.  The CUs
+// up to 11/8 workgroups per CU, or fewer than 16 key tiles.  The CUs
 // then hold one wave per SIMD for much of the call, the part is not power
 // bound, and a wave issues half as many MFMAs: 32.7 against 35.5 us for 3
 // q-tiles per head over 2048 keys (B = 2, 32 heads x 128: 192 workgroups), 70.5
-// against 73.8 us for 5 over 4608 keys at 32 x 64 (320), and 26.0 against
-// 27.4 us for 9 over 832 keys.  With 448 workgroups the 16x16x32 kernel leads
+// against 73.8 us for 5 over 4608 keys at 32 x 64 (320), 30.1
+// against 31.5 us for 11 over 1728 keys at B = 1 (352), and 26.0 against 27.4
+// us for 9 over 832 keys.  With 448 workgroups the 16x16x32 kernel leads
 // again (126.9 against 130.2 us, 7 over 4608 keys).
 inline bool small_grid(const FlashParams& p, Slots s) {
-  return !p.pair && (p.tile_start[p.n_seg] < 16 || 4 * grid_blocks(p) <= 5 * (int64_t)s.pieces);
+  return !p.pair && (p.tile_start[p.n_seg] < 16 || 8 * grid_blocks(p) <= 11 * (int64_t)s.cus);
 }
 
 // fp8 K/V in frames of whole 64-key tiles with an odd number (>= 3) of
@@ -2173,9 +2205,8 @@ inline bool small_grid(const FlashParams& p, Slots s) {
 // units in one round and 64 q-tiles in 8 ranges of 9 key tiles.  SplitPlan
 // holds both launches' split plans and their partial buffers' offsets.
 struct SplitPlan {
-  int64_t n_full[2];
-  int split[2];
-  int64_t off[2], bytes[2];
+  Split s[2];
+  int64_t off[2];
   int64_t total;
 };
 
@@ -2183,26 +2214,20 @@ inline SplitPlan plan_fp8_split_launch(int64_t B, int64_t H, int64_t nqt, int nt
   SplitPlan sp{};
   // launch 0: pair units over the first nqt - 1 q-tiles of every head
   const int64_t nu0 = B * H * (nqt - 1) / 2;
-  plan_split(nu0, ntiles, flash_slots(D, kPathFp8, true), D, 2, &sp.n_full[0], &sp.split[0]);
-  sp.bytes[0] = sp.split[0] > 1 ? workspace_bytes_for((nu0 - sp.n_full[0]) * 2, sp.split[0], D) : 0;
+  sp.s[0] = plan_split(nu0, ntiles, kPathFp8, true, D);
   // launch 1: the last q-tile of every head, one piece per slot
   const int64_t nu1 = B * H;
   const Slots s1 = flash_slots(D, kPathFp8, false);
-  sp.n_full[1] = nu1;
-  sp.split[1] = 1;
+  sp.s[1] = {nu1, 1, false};
   if (s1.slots > 0 && nu1 < s1.slots) {
     int k = (int)(s1.slots / nu1);
     k = k > kMaxSplit ? kMaxSplit : k;
     k = k > ntiles / 2 ? ntiles / 2 : k;   // pieces of >= 2 key tiles
-    if (k >= 2) {
-      sp.n_full[1] = 0;
-      sp.split[1] = k;
-    }
+    if (k >= 2) sp.s[1] = {0, k, false};
   }
-  sp.bytes[1] = sp.split[1] > 1 ? workspace_bytes_for(nu1 - sp.n_full[1], sp.split[1], D) : 0;
   sp.off[0] = 0;
-  sp.off[1] = round256(sp.bytes[0]);
-  sp.total = sp.off[1] + sp.bytes[1];
+  sp.off[1] = round256(sp.s[0].bytes(nu0, 2, D));
+  sp.total = sp.off[1] + sp.s[1].bytes(nu1, 1, D);
   return sp;
 }
 
@@ -2223,7 +2248,8 @@ extern "C" int ltx_flash_attn_workspace_size(int64_t B, int64_t Lq, int64_t H, i
     const FlashPath path = k == 4 ? kPathFp8 : (FlashPath)k;
     const bool kp = pair && k != 4 && path != kPathMasked;
     const int64_t nu = kp ? nq / 2 : nq;
-    const int64_t b = split_bytes_bound(nu, flash_slots(D, path, kp), D, kp ? 2 : 1);
+    // no call of this shape plans more than one with an unbounded key count
+    const int64_t b = plan_split(nu, 1 << 30, path, kp, D).bytes(nu, kp ? 2 : 1, D);
     need = b > need ? b : need;
   }
   // the two-launch fp8 plan for an odd q-tile count
@@ -2235,10 +2261,8 @@ extern "C" int ltx_flash_attn_workspace_size(int64_t B, int64_t Lq, int64_t H, i
   return LTX_OK;
 }
 
-// The body of both attention entry points.  `strict_ws`: a planned split
-// whose partials do not fit the workspace is an error (the no-allocation
-// entry point, whose workspace is the fixed scratch array) instead of a
-// fallback to whole q-tiles.  `seg_bs`: each segment's own batch stride (in
+// The body of the attention entry points.  A planned split whose partials do
+// not fit the workspace runs whole.  `seg_bs`: each segment's own batch stride (in
 // elements, instead of k_bs), for token-major bf16 K/V.
 static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, int64_t D,
                                int64_t q_bs, int64_t q_ls, int64_t q_hs, int64_t n_segments,
@@ -2249,7 +2273,7 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
                                int64_t sc_bs, int64_t sc_hs, int64_t frame_tokens,
                                const float* key_mask, int64_t mask_bs, const int64_t* key_lens, void* out,
                                int64_t o_bs, int64_t o_ls, int64_t o_hs, float* lse, float scale,
-                               void* workspace, int64_t workspace_bytes, bool strict_ws, void* stream,
+                               void* workspace, int64_t workspace_bytes, void* stream,
                                const int64_t* seg_bs = nullptr) {
   LTX_REQUIRE(q && out, "ltx_flash_attn_fwd: null q/out");
   LTX_REQUIRE(D == 64 || D == 128, "ltx_flash_attn_fwd: head dim %lld unsupported (64 or 128)",
@@ -2363,7 +2387,7 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
     const SplitPlan sp = plan_fp8_split_launch(B, H, p.n_qtiles, p.tile_start[n], D);
     if (sp.total <= workspace_bytes) {
       LTX_REQUIRE(al(workspace, 256), "ltx_flash_attn_fwd: workspace must be 256-byte aligned");
-      const int64_t lq0 = (int64_t)(p.n_qtiles - 1) * kBM;
+      const int64_t lq0 = (int64_t)(p.n_qtiles - 1) * kBM, nq0 = (int64_t)B * H * (p.n_qtiles - 1);
       FlashParams lp[2] = {p, p};
       lp[0].Lq = (int)lq0;
       lp[0].n_qtiles = p.n_qtiles - 1;
@@ -2375,14 +2399,12 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
       lp[1].n_qtiles = 1;
       lp[1].pair = 0;
       for (int i = 0; i < 2; ++i) {
-        lp[i].n_full = (int)sp.n_full[i];
-        lp[i].split = sp.split[i];
-        if (sp.split[i] > 1) {
-          const int64_t tail = (i == 0 ? 2 * ((int64_t)B * H * lp[0].n_qtiles / 2 - sp.n_full[0])
-                                       : (int64_t)B * H - sp.n_full[1]);
-          lp[i].part_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + sp.off[i]);
-          lp[i].part_o = reinterpret_cast<uint16_t*>(lp[i].part_ml + tail * sp.split[i] * kBM * 2);
-        }
+        lp[i].n_full = (int)sp.s[i].n_full;
+        lp[i].split = sp.s[i].n;
+        lp[i].part_f32 = sp.s[i].f32;
+        const int64_t rows = sp.s[i].rows(i == 0 ? nq0 / 2 : (int64_t)B * H, i == 0 ? 2 : 1);
+        lp[i].part_ml = reinterpret_cast<float*>(static_cast<char*>(workspace) + sp.off[i]);
+        lp[i].part_o = lp[i].part_ml + 2 * rows;
         const int rc = D == 128 ? launch_flash_pipe<128, kFp8>(lp[i], st) : launch_flash_pipe<64, kFp8>(lp[i], st);
         if (rc != LTX_OK) return rc;
       }
@@ -2400,26 +2422,18 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
     p.pair = path != kPathMasked && (!fp8 || frame_tokens % kBN == 0) && p.n_qtiles % 2 == 0 ? 1 : 0;
     const int64_t nu = p.pair ? nq / 2 : nq;
     const int per_unit = p.pair ? 2 : 1;
-    int64_t n_full = nu;
-    int split = 1;
+    Split sp{nu, 1, false};
     if (workspace != nullptr) {
-      plan_split(nu, p.tile_start[n], flash_slots(D, path, p.pair != 0), D, per_unit, &n_full, &split);
-      if (split > 1 && workspace_bytes_for((nu - n_full) * per_unit, split, D) > workspace_bytes) {
-        LTX_REQUIRE(!strict_ws,
-                    "ltx_flash_attn_fwd_noalloc: this call's split partials need %lld bytes, more than the "
-                    "%lld-byte scratch array",
-                    (long long)workspace_bytes_for((nu - n_full) * per_unit, split, D), (long long)workspace_bytes);
-        n_full = nu;
-        split = 1;
-      }
+      sp = plan_split(nu, p.tile_start[n], path, p.pair != 0, D);
+      if (sp.bytes(nu, per_unit, D) > workspace_bytes) sp = {nu, 1, false};
     }
-    p.n_full = (int)n_full;
-    p.split = split;
-    if (split > 1) {
+    p.n_full = (int)sp.n_full;
+    p.split = sp.n;
+    p.part_f32 = sp.f32;
+    if (sp.n > 1) {
       LTX_REQUIRE(al(workspace, 256), "ltx_flash_attn_fwd: workspace must be 256-byte aligned");
-      const int64_t tail = (nu - n_full) * per_unit;
       p.part_ml = static_cast<float*>(workspace);
-      p.part_o = reinterpret_cast<uint16_t*>(p.part_ml + tail * split * kBM * 2);
+      p.part_o = p.part_ml + 2 * sp.rows(nu, per_unit);
     }
   }
   switch (path) {
@@ -2454,7 +2468,7 @@ extern "C" int ltx_flash_attn_fwd(const void* q, int64_t B, int64_t Lq, int64_t 
   return flash_attn_fwd_impl(q, B, Lq, H, D, q_bs, q_ls, q_hs, n_segments, k_ptrs, v_ptrs, seg_lens, k_bs,
                              k_ls, k_hs, v_bs, v_ls, v_hs, v_ds, kv_dtype, k_scales, v_scales, sc_bs, sc_hs,
                              frame_tokens, key_mask, mask_bs, key_lens, out, o_bs, o_ls, o_hs, lse, scale,
-                             workspace, workspace_bytes, false, stream);
+                             workspace, workspace_bytes, stream);
 }
 
 extern "C" int ltx_flash_attn_fwd_plain(const void* q, int64_t B, int64_t Lq, int64_t H, int64_t D, int64_t q_bs,
@@ -2467,19 +2481,20 @@ extern "C" int ltx_flash_attn_fwd_plain(const void* q, int64_t B, int64_t Lq, in
   LTX_REQUIRE(n_segments == 0 || seg_bs != nullptr, "ltx_flash_attn_fwd_plain: null segment batch strides");
   return flash_attn_fwd_impl(q, B, Lq, H, D, q_bs, q_ls, q_hs, n_segments, k_ptrs, v_ptrs, seg_lens, 0, kv_ls, kv_hs,
                              0, kv_ls, kv_hs, 1, LTX_BF16, nullptr, nullptr, 0, 0, 0, nullptr, 0, nullptr, out, o_bs,
-                             o_ls, o_hs, lse, scale, workspace, workspace_bytes, false, stream, seg_bs);
+                             o_ls, o_hs, lse, scale, workspace, workspace_bytes, stream, seg_bs);
 }
 
 // ---------------------------------------------------------------------------
 // No-allocation variant: the split partials live in a fixed device array.
 //
 // `scratch` holds the partial results of the split tail q-tiles (per piece:
-// 128 rows of (max, sum) in float32 and an O row in bf16).  split_limit keeps
-// every plan's partials within the array (the fp8 two-launch plan keeps both
-// launches' partials in it and is taken only when they fit).  Every piece
-// writes its whole partial before the combine kernel reads it, so nothing
-// needs clearing between calls.  Each
-// device holds its own copy of the array for the life of the process; its
+// 128 rows of (max, sum) in float32 and an O row in bf16 or float32): 384
+// float32 pieces at D = 128 or 768 at D = 64, and every bf16 plan of one launch
+// (at most 512 pieces at D = 128).  A float32 plan that needs more runs whole,
+// and the fp8 two-launch plan, which keeps both launches' partials, is taken
+// only where they fit (else one launch).  Every piece writes its whole partial
+// before the combine kernel reads it, so nothing needs clearing between calls.
+// Each device holds its own copy of the array for the life of the process; its
 // device address is looked up once per device (hipGetSymbolAddress) and
 // only that address is handed to kernels.  Calls that overlap in time on one
 // device share the array and race.
@@ -2527,5 +2542,5 @@ extern "C" int ltx_flash_attn_fwd_noalloc(const void* q, int64_t B, int64_t Lq, 
   return flash_attn_fwd_impl(q, B, Lq, H, D, q_bs, q_ls, q_hs, n_segments, k_ptrs, v_ptrs, seg_lens, k_bs,
                              k_ls, k_hs, v_bs, v_ls, v_hs, v_ds, kv_dtype, k_scales, v_scales, sc_bs, sc_hs,
                              frame_tokens, key_mask, mask_bs, key_lens, out, o_bs, o_ls, o_hs, lse, scale, ws,
-                             kScratchBytes, true, stream);
+                             kScratchBytes, stream);
 }

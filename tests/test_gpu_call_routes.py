@@ -3,13 +3,14 @@ reference: plain caches in strides and alignments that are attended in place
 or concatenated, key-range splits of partly filled grids, norm rows without
 RoPE tables, and the timestep MLPs with and without the row kernel."""
 import contextlib
+import ctypes
 import math
 
 import pytest
 import torch
 
 import taomate_amd as T
-from taomate_amd import dit, kernels
+from taomate_amd import _native, dit, kernels
 from taomate_amd.kernels import KVSegment
 
 from .helpers import gen, randn
@@ -92,6 +93,69 @@ def test_split_plans(dev, layout, B, H, D, qtiles, keys):
         sl = slice(h, h + 1)
         ref = _attend64(q[:, :, sl].cpu(), k[:, :, sl].cpu(), v[:, :, sl].cpu())
         assert (out[:, :, sl].double().cpu() - ref).abs().max().item() <= _bound(v) + 2.0 ** -8 * ref.abs().max().item()
+
+
+def _fp8_cache(k, v, frame, dev):
+    """fp8 codes and scales of K and V, and the values they hold."""
+    B, n, H, D = k.shape
+    kc, vc = (torch.empty(B, n, H, D, dtype=torch.uint8, device=dev) for _ in range(2))
+    ks, vs = (torch.empty(B, H, n // frame, device=dev) for _ in range(2))
+    kernels.kv_append_fp8_pair(k, kc, ks, v, vc, vs, frame)
+    value = lambda c, s: (c.view(torch.float8_e4m3fn).double()
+                          * s.double().transpose(1, 2).repeat_interleave(frame, 1)[..., None])
+    return KVSegment(kc, vc, ks, vs), value(kc, ks), value(vc, vs)
+
+
+def _whole(q, seg, out, frame):
+    """The same call without a workspace: every q-tile runs whole, in float32 sums."""
+    k, v = seg.k, seg.v
+    fp8 = seg.k_scales is not None
+    keep = [_native.ptr_array([t.data_ptr()]) for t in (k, v)] + [_native.i64_array([k.shape[1]])] + \
+        [_native.ptr_array([t.data_ptr()]) if fp8 else None for t in (seg.k_scales, seg.v_scales)]
+    kp, vp, lens, ksp, vsp = (None if a is None else ctypes.cast(a, ctypes.c_void_p) for a in keep)
+    _native.call("ltx_flash_attn_fwd", q.data_ptr(), *q.shape, *q.stride()[:3], 1, kp, vp, lens, *k.stride()[:3],
+                 *v.stride(), 2 if fp8 else 1, ksp, vsp, *(seg.k_scales.stride()[:2] if fp8 else (0, 0)), frame, None, 0,
+                 None, out.data_ptr(), *out.stride()[:3], None, 0.0, None, 0,
+                 torch.cuda.current_stream().cuda_stream)
+
+
+@pytest.mark.parametrize("layout,B,Lq,H,D,keys", [
+    ("key", 1, 620, 32, 128, 4000), ("key", 2, 300, 32, 64, 5000), ("key", 2, 620, 32, 64, 5000),
+    ("key", 1, 1370, 32, 128, 7000), ("token", 2, 620, 32, 128, 4000), ("token", 1, 300, 32, 64, 2600),
+    ("token", 2, 512, 32, 64, 2000), ("token", 2, 1152, 32, 64, 1152), ("token", 1, 2423, 32, 128, 1152),
+    ("fp8", 1, 620, 32, 64, 1650), ("fp8", 2, 300, 32, 128, 2640), ("fp8", 2, 620, 32, 128, 3300),
+    ("fp8", 1, 1370, 32, 64, 4950)])
+def test_split_keeps_float32_sums(dev, layout, B, Lq, H, D, keys):
+    """Tails that are split with float32 partials, one case per branch of the
+    launch plan: the error against float64 is the whole q-tiles' (bf16
+    partials of all rows make it 1.22 times that).  Both share P's rounding
+    and the output's; over the 1e5 and more values compared, what is left
+    differs by well under 1 %."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(keys + Lq)
+    r = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+    q, k, v = r(B, Lq, H, D), r(B, keys, H, D), r(B, keys, H, D)
+    frame = 330 if layout == "fp8" else 0
+    if layout == "fp8":
+        seg, k, v = _fp8_cache(k, v, frame, dev)
+    elif layout == "key":
+        store = torch.zeros(B, H, D, -(-keys // 8) * 8, dtype=torch.bfloat16, device=dev)
+        store[..., :keys] = v.permute(0, 2, 3, 1)
+        seg = KVSegment(k, store[..., :keys].permute(0, 3, 1, 2))
+    else:
+        seg = KVSegment(k, v)
+    out, whole = torch.empty_like(q), torch.empty_like(q)
+    kernels.flash_attn(q, [seg], out, frame_tokens=frame)
+    _whole(q, seg, whole, frame)
+    torch.cuda.synchronize()
+    assert not torch.equal(out, whole)   # the plan does split
+    err = [0.0, 0.0]
+    for b, h in ((0, 0), (B - 1, H - 1), (0, H // 2), (B - 1, 5)):
+        p = ((q[b, :, h].double() @ k[b, :, h].double().t().contiguous()) / math.sqrt(D)).softmax(-1)
+        ref = p @ v[b, :, h].double()
+        for i, o in enumerate((out, whole)):
+            err[i] += (o[b, :, h].double() - ref).square().sum().item()
+    assert math.sqrt(err[0] / err[1]) <= 1.02
 
 
 @pytest.mark.parametrize("B,L,H,D", [(2, 1, 8, 64), (1, 33, 32, 128), (2, 75, 32, 64)])
