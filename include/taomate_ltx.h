@@ -275,10 +275,14 @@ int ltx_flash_attn_fwd_plain(const void* q, int64_t B, int64_t Lq, int64_t H, in
  *   sufficient workspace; the split partials go to a fixed device array of
  *   LTX_NOALLOC_SCRATCH_BYTES inside the library (one per device, kept until
  *   the process ends).  Allocates nothing: no hipMalloc / hipFree, no
- *   allocating library call.  Both entry points plan splits whose partials fit
- *   that array, so the results are the same.  Calls that overlap in time on
- *   one device share the array and race: serialise them (one stream, or
- *   events).
+ *   allocating library call.  The same launch plan as ltx_flash_attn_fwd
+ *   where its partials fit the array, and then the same results bit for bit.
+ *   Where they do not (float32 partials of more than 384 pieces of 128 x 128 or
+ *   768 of 128 x 64; fp8 K/V in frames of whole 64-key tiles at an odd q-tile
+ *   count, whose two launches may need up to 33 MiB: 384 or 640 queries at B = 2
+ *   and 32 heads x 128) the call runs without that split: at least as exact,
+ *   rounded differently.  Calls that overlap in time on one device share the
+ *   array and race: serialise them (one stream, or events).
  */
 #define LTX_NOALLOC_SCRATCH_BYTES (25ll << 20)
 int ltx_flash_attn_fwd_noalloc(const void* q, int64_t B, int64_t Lq, int64_t H, int64_t D,

@@ -101,3 +101,22 @@ def test_noalloc_fp8_pair_matches_workspace_entry_point(dev, first, second):
         assert torch.equal(out, ref_out), f"call {i}: noalloc output differs from the workspace entry point"
         if i == 0:
             assert_bf16_close(out, _ref_attn(q.cpu(), K, V), "noalloc fp8 vs the dequantised cache")
+
+
+@pytest.mark.parametrize("Lq", [384, 640])
+def test_noalloc_fp8_where_two_launches_do_not_fit(dev, Lq):
+    """Three and five q-tiles per head at B = 2 and 32 heads: the two launches'
+    partials exceed the scratch array, so the call runs as one launch."""
+    B, H, D, frame = 2, 32, 128, 384
+    g = gen(23)
+    segs, K, V = _fp8_segments(dev, B, H, D, [384, 768], frame, g)
+    q = randn((B, Lq, H, D), g, torch.bfloat16).to(dev)
+    out, ws = (torch.full((B, Lq, H, D), float("nan"), dtype=torch.bfloat16, device=dev) for _ in range(2))
+    kernels.flash_attn(q, segs, out, frame_tokens=frame, noalloc=True)
+    kernels.flash_attn(q, segs, ws, frame_tokens=frame)
+    torch.cuda.synchronize()
+    ref = _ref_attn(q.cpu(), K, V)
+    for o in (out, ws):
+        assert_bf16_close(o, ref, "fp8 vs the dequantised cache")
+    err = [(o.float().cpu() - ref).norm() for o in (out, ws)]
+    assert err[0] <= 1.02 * err[1]   # whole q-tiles: no rounding between the two
