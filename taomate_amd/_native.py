@@ -99,13 +99,16 @@ def load() -> ctypes.CDLL:
             lib = ctypes.CDLL(str(path))
         except OSError as e:
             raise NativeLibraryError(f"cannot load {path}: {e}") from e
-        for name, argtypes in SIGNATURES.items():
-            fn = getattr(lib, name)
-            fn.argtypes = argtypes
-            fn.restype = ctypes.c_char_p if name == "ltx_last_error" else ctypes.c_int
-        ver = lib.ltx_abi_version()
-        if ver != ABI_VERSION:
-            raise NativeLibraryError(f"{path}: ABI version {ver}, expected {ABI_VERSION}")
+        try:
+            ver = lib.ltx_abi_version()
+            if ver != ABI_VERSION:
+                raise NativeLibraryError(f"{path}: ABI version {ver}, expected {ABI_VERSION}")
+            for name, argtypes in SIGNATURES.items():
+                fn = getattr(lib, name)
+                fn.argtypes = argtypes
+                fn.restype = ctypes.c_char_p if name == "ltx_last_error" else ctypes.c_int
+        except AttributeError as e:   # an ABI keeps its version when entry points are added to it
+            raise NativeLibraryError(f"{path} lacks an entry point, build it again: {e}") from e
         _lib = lib
         return lib
 

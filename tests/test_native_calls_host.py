@@ -1,5 +1,6 @@
 """The native call module's argument checks, without a GPU: what the wrappers
 refuse and with which error, and how long they hold what they are given."""
+import ctypes
 import weakref
 
 import pytest
@@ -78,3 +79,27 @@ def test_rope_tables_are_held_for_the_call(side):
     assert "unsupported dtype" not in str(e.value)
     assert eps.alive == [True, True]
     assert [r() for r in tab.refs] == [None, None]   # and no longer than the call
+
+
+class _Entry:
+    def __init__(self, value):
+        self.value = value
+
+    def __call__(self):
+        return self.value
+
+
+@pytest.mark.parametrize("have,message", [
+    ({"ltx_abi_version": 2, "ltx_last_error": b""}, "ltx_rope_table"),         # an older library of this ABI
+    ({"ltx_abi_version": 1}, "ABI version 1, expected 2"),
+    ({}, "ltx_abi_version"),                                                   # another library altogether
+])
+def test_a_library_without_the_entry_points_is_refused(monkeypatch, have, message):
+    lib = type("Lib", (), {})()
+    for name, value in have.items():
+        setattr(lib, name, _Entry(value))
+    monkeypatch.setattr(_native, "_lib", None)
+    monkeypatch.setattr(ctypes, "CDLL", lambda path: lib)
+    with pytest.raises(_native.NativeLibraryError, match=message):
+        _native.load()
+    assert _native._lib is None
