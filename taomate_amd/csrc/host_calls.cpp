@@ -516,6 +516,8 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     Py_RETURN_NONE;
   } catch (const Refused& r) {
     if (r.type != nullptr) PyErr_SetString(r.type, r.msg.c_str());
+  } catch (const c10::IndexError& e) {
+    PyErr_SetString(PyExc_IndexError, e.what_without_backtrace());
   } catch (const std::exception& e) {
     PyErr_SetString(PyExc_RuntimeError, e.what());
   }

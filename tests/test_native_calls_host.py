@@ -81,6 +81,14 @@ def test_rope_tables_are_held_for_the_call(side):
     assert [r() for r in tab.refs] == [None, None]   # and no longer than the call
 
 
+def test_a_segment_without_a_token_dim_is_an_index_error():
+    with FakeTensorMode():
+        rows = torch.empty(1, 4, 1, 64, dtype=torch.bfloat16, device="cuda")
+    flat = torch.zeros(64, dtype=torch.bfloat16)
+    with pytest.raises(IndexError):
+        kernels.flash_attn(rows, [KVSegment(flat, flat)], rows)
+
+
 class _Entry:
     def __init__(self, value):
         self.value = value
