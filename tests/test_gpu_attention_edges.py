@@ -57,3 +57,80 @@ def test_pipelined_edges(dev, D, Lq, lens, vlayout):
         assert (out.double().cpu() - ref).abs().max().item() <= bound
         assert torch.isnan(store[..., :off]).all() and torch.isnan(store[..., off + H * D:]).all()
         assert (lse.double().cpu() - s.logsumexp(-1)).abs().max().item() <= 2.0 ** -9
+
+
+def _segments(dev, k, v, lens, layout):
+    """K and V [B, n, H, D] cut into spans of one store, each at an 8-token offset."""
+    B, _, H, D = k.shape
+    cap = sum(-(-m // 8) * 8 for m in lens)
+    ka = torch.zeros(B, cap, H, D, dtype=torch.bfloat16, device=dev)
+    va = torch.zeros(B, H, D, cap, dtype=torch.bfloat16, device=dev).permute(0, 3, 1, 2) if layout == "key" \
+        else torch.zeros_like(ka)
+    segs, pos, at = [], 0, 0
+    for m in lens:
+        ka[:, pos:pos + m], va[:, pos:pos + m] = k[:, at:at + m], v[:, at:at + m]
+        segs.append(KVSegment(ka[:, pos:pos + m], va[:, pos:pos + m]))
+        at += m
+        pos += -(-m // 8) * 8
+    return segs
+
+
+@pytest.mark.parametrize("layout,form", [("key", "plain"), ("key", "lens"), ("token", "plain")])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Lq", [257, 273, 289])
+def test_single_tile_workgroups(dev, D, Lq, layout, form):
+    """Three q-tiles per head of 128 heads over 19 key tiles: the 4-wave
+    workgroups of the 16x16x32 body, whole, with ragged queries and segments,
+    output rows of 16- and 8-byte alignment, the log-sum-exp and per-row key
+    counts, against float64 on a few heads."""
+    B, H, lens = 2, 64, (9, 63, 1000, 1)
+    g = torch.Generator(device=dev)
+    g.manual_seed(Lq + D)
+    r = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+    n = sum(lens)
+    q, k, v = r(B, Lq, H, D), r(B, n, H, D), r(B, n, H, D)
+    segs = _segments(dev, k, v, lens, layout)
+    counts = [n, 700] if form == "lens" else [n, n]
+    lse = torch.empty(B, H, Lq, dtype=torch.float32, device=dev)
+    for off in (0, 4):
+        store = torch.full((B, Lq, H * D + 8), float("nan"), dtype=torch.bfloat16, device=dev)
+        out = store[..., off:off + H * D].view(B, Lq, H, D)
+        kernels.flash_attn(q, segs, out, lse=lse, key_lens=counts if form == "lens" else None)
+        torch.cuda.synchronize()
+        assert torch.isnan(store[..., :off]).all() and torch.isnan(store[..., off + H * D:]).all()
+        assert not torch.isnan(out).any()
+        for b, h in ((0, 0), (0, 37), (1, 1), (1, H - 1)):
+            m = counts[b]
+            s = q[b, :, h].double() @ k[b, :m, h].double().t().contiguous() / math.sqrt(D)
+            ref = s.softmax(-1) @ v[b, :m, h].double()
+            # P, the output and the ratio of the rounded P's to the row sum (half a bf16 ulp each)
+            assert (out[b, :, h].double() - ref).abs().max().item() <= 3 * 2.0 ** -9 * v.abs().max().item()
+            assert (lse[b, h].double() - s.logsumexp(-1)).abs().max().item() <= 2.0 ** -9
+
+
+@pytest.mark.parametrize("layout", ["key", "token"])
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Lq", [100, 256, 300])
+def test_nothing_of_an_earlier_tile_is_read(dev, D, Lq, layout):
+    """Partial tiles after a call that leaves NaN in every tile buffer of the
+    LDS: the keys past a segment's end have weight 0, so their V must be
+    finite (rows past it load zeros, or repeat a chunk of the segment)."""
+    B, H, lens = 2, 32, (9, 63, 65, 130, 1)
+    nan = torch.full((B, 256, H, D), float("nan"), dtype=torch.bfloat16, device=dev)
+    g = torch.Generator(device=dev)
+    g.manual_seed(D)
+    r = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+    n = sum(lens)
+    q, k, v = r(B, Lq, H, D), r(B, n, H, D), r(B, n, H, D)
+    segs, bad = _segments(dev, k, v, lens, layout), _segments(dev, nan, nan, (256,), layout)
+    fill_q, out = r(B, 1152, H, D), torch.empty_like(q)
+    fill_out = torch.empty_like(fill_q)
+    kernels.flash_attn(fill_q, bad, fill_out)
+    kernels.flash_attn(q, segs, out)
+    torch.cuda.synchronize()
+    assert torch.isnan(fill_out).all()
+    for b, h in ((0, 0), (1, H - 1)):
+        s = q[b, :, h].double() @ k[b, :, h].double().t().contiguous() / math.sqrt(D)
+        ref = s.softmax(-1) @ v[b, :, h].double()
+        assert (out[b, :, h].double() - ref).abs().max().item() <= 3 * 2.0 ** -9 * v.abs().max().item()
+    assert not torch.isnan(out).any()
