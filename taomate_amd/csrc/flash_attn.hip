@@ -1822,12 +1822,20 @@ __device__ __forceinline__ void flash_mfma32_body(const FlashParams& p) {
           }
         }
       }
-      // the slot's order: MFMA, fragment read, exp, other vector work (fp8 at
-      // 1152 x 6912: 236.1 -> 234.4 us, and the D = 128 instances no longer spill)
-      __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);
-      __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+      // the slot's order at D = 128: MFMA, fragment read, exp, other vector work.
+      // Medians of four alternating runs, without and with it: fp8 1152 x 6912
+      // 237.7 and 234.4 us, 1728 x 10368 523.6 and 514.7, in 330-token frames
+      // 990 x 5940 234.5 and 229.8 (another box: 240.3 and 238.5, 524.6 and 521.4,
+      // 236.7 and 233.0); spilled VGPRs of the fp8 kernels: pair 1 and 0,
+      // 4-wave 2 and 0, framed 12 and 6.  At D = 64 the compiler's order is the
+      // faster one (fp8 1152 x 6912 167.5 against 169.0 us, bf16 300 x 4500 48.4
+      // against 48.9).
+      if constexpr (D == 128) {
+        __builtin_amdgcn_sched_group_barrier(0x8, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x400, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x2, 3, 0);
+      }
       __builtin_amdgcn_sched_barrier(0);
     }
   };
