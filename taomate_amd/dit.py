@@ -93,13 +93,22 @@ def _is_plain(m: nn.Module, cls: type) -> bool:
                      or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks))
 
 
+_autocast, _function_modes, _dispatch_modes = (torch.is_autocast_enabled, torch._C._len_torch_function_stack,
+                                               torch._C._len_torch_dispatch_stack)
+_transform, _trace = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
+
+
 def _is_eager() -> bool:
     """Whether an op on plain tensors would run as it is written: no gradients,
     autocast, forward-mode level, function transform, torch function or
     dispatch mode, trace or compilation sees it."""
-    return not (torch.is_grad_enabled() or torch.is_autocast_enabled("cuda") or forward_ad._current_level >= 0
-                or torch._C._functorch.peek_interpreter_stack() is not None or torch._C._len_torch_function_stack()
-                or torch._C._len_torch_dispatch_stack() or torch.jit.is_tracing() or torch.compiler.is_compiling())
+    return not (torch.is_grad_enabled() or _autocast("cuda") or forward_ad._current_level >= 0
+                or _transform() is not None or _function_modes() or _dispatch_modes()
+                or _trace() is not None or torch.compiler.is_compiling())
+
+
+def _is_operand(t: torch.Tensor, x: torch.Tensor) -> bool:
+    return type(t) in (nn.Parameter, torch.Tensor) and t.dtype == x.dtype and t.is_contiguous() and t.device == x.device
 
 
 def _row_linear(lin: nn.Module, x: torch.Tensor, act: Optional[nn.Module] = None) -> torch.Tensor:
@@ -112,10 +121,8 @@ def _row_linear(lin: nn.Module, x: torch.Tensor, act: Optional[nn.Module] = None
         if (type(x) is torch.Tensor and x.dtype == torch.bfloat16 and x.dim() == 2
                 and 1 <= x.shape[0] <= kernels.SKINNY_MAX_ROWS and x.shape[1] <= kernels.SKINNY_MAX_K
                 and x.shape[1] % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
-                and all(t is None or type(t) in (nn.Parameter, torch.Tensor) and t.dtype == x.dtype
-                        and t.device == x.device and t.is_contiguous() for t in (w, b))
-                and w.dim() == 2 and w.shape[1] == x.shape[1] and w.data_ptr() % 16 == 0
-                and (b is None or b.shape == w.shape[:1])):
+                and _is_operand(w, x) and w.dim() == 2 and w.shape[1] == x.shape[1] and w.data_ptr() % 16 == 0
+                and (b is None or _is_operand(b, x) and b.shape == w.shape[:1])):
             return kernels.skinny_linear(x, w, b, silu=act is not None)
     return lin(x if act is None else act(x))
 
