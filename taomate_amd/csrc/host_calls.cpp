@@ -296,7 +296,9 @@ void kv_append_fp8_pair(PyObject* const* a) {
 // merge of its partials as separate launches, so it holds the workspace's lock
 // until both are in the stream: threads that share a stream (PyTorch's all start
 // on one) take turns.  The lock is taken with the GIL released and given back
-// before the GIL is taken again, so neither waits for the other.  The map is
+// before the GIL is taken again, so neither waits for the other.  A captured
+// graph keeps its stream's workspace: graphs captured on one stream must not
+// replay at the same time.  The map is
 // kept for the life of the process (never destroyed: the allocator may be gone
 // by then), and its entries never move.
 struct Workspace {
