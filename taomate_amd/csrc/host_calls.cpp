@@ -296,11 +296,14 @@ void kv_append_fp8_pair(PyObject* const* a) {
 // merge of its partials as separate launches, so it holds the workspace's lock
 // until both are in the stream: threads that share a stream (PyTorch's all start
 // on one) take turns.  The lock is taken with the GIL released and given back
-// before the GIL is taken again, so neither waits for the other.  A captured
-// graph keeps its stream's workspace: graphs captured on one stream must not
-// replay at the same time.  The map is
+// before the GIL is taken again, so neither waits for the other.  The map is
 // kept for the life of the process (never destroyed: the allocator may be gone
 // by then), and its entries never move.
+//
+// A call that is captured into a graph takes a tensor of its own instead, from
+// the graph's memory pool: replays keep its address, which must neither be freed
+// when a later call grows the stream's workspace nor be shared with other graphs
+// or eager calls that run beside them.
 struct Workspace {
   std::mutex mu;
   at::Tensor buf;
@@ -310,6 +313,12 @@ Workspace& workspace(const at::Tensor& q, void* stream) {
   static auto* kept = new std::map<std::pair<int, void*>, Workspace>;
   std::lock_guard<std::mutex> lock(mu);
   return (*kept)[{q.device().index(), stream}];
+}
+
+bool capturing(void* stream) {
+  hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+  return stream != nullptr && hipStreamIsCapturing(static_cast<hipStream_t>(stream), &st) == hipSuccess &&
+         st != hipStreamCaptureStatusNone;
 }
 
 PyObject *str_k, *str_v, *str_ks, *str_vs;
@@ -437,15 +446,18 @@ void flash_attn(PyObject* const* a) {
   call("ltx_flash_attn_workspace_size", api.flash_attn_workspace_size, B, Lq, H, D, &need);
   released(own_bs ? "ltx_flash_attn_fwd_plain" : "ltx_flash_attn_fwd", [&] {
     std::unique_lock<std::mutex> lock;
-    void* wsp = nullptr;
-    int64_t ws_bytes = 0;
-    if (need > 0) {
+    at::Tensor buf;
+    const auto bytes = [&] { return at::empty({need}, q.options().dtype(at::kByte)); };
+    if (need > 0 && capturing(st)) {
+      buf = bytes();
+    } else if (need > 0) {
       Workspace& ws = workspace(q, st);
       lock = std::unique_lock<std::mutex>(ws.mu);
-      if (!ws.buf.defined() || ws.buf.numel() < need) ws.buf = at::empty({need}, q.options().dtype(at::kByte));
-      wsp = ws.buf.data_ptr();
-      ws_bytes = ws.buf.numel();
+      if (!ws.buf.defined() || ws.buf.numel() < need) ws.buf = bytes();
+      buf = ws.buf;
     }
+    void* wsp = buf.defined() ? buf.data_ptr() : nullptr;
+    const int64_t ws_bytes = buf.defined() ? buf.numel() : 0;
     if (!own_bs) return general(api.flash_attn_fwd, wsp, ws_bytes, st);
     return api.flash_attn_fwd_plain(ptr(&q), B, Lq, H, D, q.stride(0), q.stride(1), q.stride(2), (int64_t)n, kp, vp,
                                     lens, seg_bs, k0.stride(1), k0.stride(2), ptr(&out), out.stride(0),

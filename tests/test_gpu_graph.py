@@ -64,3 +64,54 @@ def test_step_graph_replays_match_eager(dev):
         for name, a, b in zip(("q", "k slots", "v slots", "out"), outs, eager):
             assert torch.equal(a, b), f"replay {rep}: {name} differs from the eager step"
         lin[0].add_(0)       # eager work on the inputs between replays
+
+
+def test_graphs_own_their_split_workspace(dev):
+    """Two graphs captured on one stream that also ran the calls eagerly, then a
+    larger eager call there, which grows the stream's workspace, and tensors in
+    whatever memory that freed: replays, also of both graphs at once, neither
+    touch those tensors nor each other's partial results."""
+    g = torch.Generator(device=dev)
+    g.manual_seed(9)
+    r = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+
+    def call(B, Lq, H, D, n):
+        q, k, v = r(B, Lq, H, D), r(B, n, H, D), r(B, n, H, D)
+        out = torch.empty_like(q)
+        return (lambda: kernels.flash_attn(q, [KVSegment(k, v)], out)), out
+
+    small, big = [call(2, 75, 32, 64, 1152), call(1, 75, 32, 128, 2000)], call(1, 620, 32, 128, 4000)
+    stream, other = torch.cuda.Stream(), torch.cuda.Stream()
+    graphs, want = [], []
+    with torch.cuda.stream(stream):
+        for fn, out in small:
+            fn()
+            stream.synchronize()
+            want.append(out.clone())
+    torch.cuda.synchronize()
+    for fn, _ in small:
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            fn()
+        graphs.append(graph)
+    with torch.cuda.stream(stream):
+        big[0]()
+        stream.synchronize()
+        big_want = big[1].clone()
+        guard = [torch.full((n << 18,), 7, dtype=torch.uint8, device=dev) for n in (1, 2, 4, 8, 16, 32, 64) * 2]
+    torch.cuda.synchronize()
+    for rep in range(4):
+        for _, out in small:
+            out.fill_(float("nan"))
+        big[1].fill_(float("nan"))
+        torch.cuda.synchronize()
+        with torch.cuda.stream(stream):
+            graphs[0].replay()
+            big[0]()
+        with torch.cuda.stream(other):
+            graphs[1].replay()
+        torch.cuda.synchronize()
+        assert torch.equal(big[1], big_want), rep
+        for (_, out), w in zip(small, want):
+            assert torch.equal(out, w), rep
+        assert all((t == 7).all() for t in guard), rep
