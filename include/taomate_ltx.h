@@ -312,6 +312,8 @@ int ltx_flash_attn_workspace_size(int64_t B, int64_t Lq, int64_t H, int64_t D, i
  *   16-byte aligned.  silu != 0 applies SiLU to x first (float32, rounded to
  *   bf16).
  */
+#define LTX_SKINNY_MAX_ROWS 8
+#define LTX_SKINNY_MAX_K 4096
 int ltx_skinny_linear(int64_t M, int64_t N, int64_t K, const void* x, int64_t x_ls, int silu,
                       const void* w, int64_t w_ls, const void* bias, void* y, int64_t y_ls,
                       void* stream);

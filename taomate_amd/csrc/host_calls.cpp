@@ -13,6 +13,11 @@
 #include <Python.h>
 
 #include <ATen/ATen.h>
+#include <ATen/PythonTorchFunctionTLS.h>
+#include <ATen/autocast_mode.h>
+#include <c10/core/GradMode.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -518,6 +523,50 @@ void skinny_linear(PyObject* const* a) {
        (int)truth(a[4]), ptr(&w), w.stride(0), ptr(bias), ptr(&y), y.stride(0), stream_of(x));
 }
 
+// is_eager(): whether an op on plain tensors would run as it is written, as far
+// as the thread's state tells: no gradients, autocast, torch function or dispatch
+// mode, function transform or trace (the last two and dispatch modes add keys to
+// the thread's included set).
+PyObject* is_eager(PyObject*, PyObject*) {
+  const auto tls = c10::impl::tls_local_dispatch_key_set();
+  return PyBool_FromLong(!c10::GradMode::is_enabled() && !at::autocast::is_autocast_enabled(at::kCUDA) &&
+                         at::impl::PythonTorchFunctionTLS::stack_len() == 0 &&
+                         c10::impl::TorchDispatchModeTLS::stack_len() == 0 &&
+                         (tls.included_ - c10::default_included_set).empty());
+}
+
+// row_operands(x, weight, bias): whether skinny_linear takes them, and they are
+// tensors or parameters without a subclass.
+PyObject* row_operands(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
+  if (nargs != 3) {
+    PyErr_Format(PyExc_TypeError, "expected 3 arguments, got %zd", nargs);
+    return nullptr;
+  }
+  auto plain = [&](PyObject* o) {
+    return THPVariable_CheckExact(o) && THPVariable_Unpack(o).layout() == at::kStrided &&
+           THPVariable_Unpack(o).scalar_type() == at::kBFloat16 && !THPVariable_Unpack(o).is_neg();
+  };
+  bool ok = false;
+  try {
+    ok = plain(args[0]) && plain(args[1]) && (args[2] == Py_None || plain(args[2]));
+    if (ok) {
+      const at::Tensor &x = THPVariable_Unpack(args[0]), &w = THPVariable_Unpack(args[1]);
+      auto aligned = [](const at::Tensor& t) { return (uintptr_t)t.data_ptr() % 16 == 0; };
+      ok = x.is_cuda() && x.dim() == 2 && x.size(0) >= 1 && x.size(0) <= LTX_SKINNY_MAX_ROWS && x.size(1) >= 8 &&
+           x.size(1) <= LTX_SKINNY_MAX_K && x.size(1) % 8 == 0 && x.stride(1) == 1 && x.stride(0) % 8 == 0 &&
+           aligned(x) && w.dim() == 2 && w.size(1) == x.size(1) && w.is_contiguous() && w.device() == x.device() &&
+           aligned(w);
+      if (ok && args[2] != Py_None) {
+        const at::Tensor& b = THPVariable_Unpack(args[2]);
+        ok = b.dim() == 1 && b.size(0) == w.size(0) && b.is_contiguous() && b.device() == x.device();
+      }
+    }
+  } catch (const std::exception&) {
+    ok = false;  // a tensor without storage
+  }
+  return PyBool_FromLong(ok);
+}
+
 // ------------------------------------------------------------------- bindings
 template <void (*Fn)(PyObject* const*), Py_ssize_t N>
 PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
@@ -579,6 +628,8 @@ PyMethodDef methods[] = {
     {"flash_attn", (PyCFunction)(void*)&entry<flash_attn, 10>, METH_FASTCALL, nullptr},
     {"skinny_linear", (PyCFunction)(void*)&entry<skinny_linear, 5>, METH_FASTCALL, nullptr},
     {"adaln", (PyCFunction)(void*)&entry<adaln, 8>, METH_FASTCALL, nullptr},
+    {"is_eager", is_eager, METH_NOARGS, nullptr},
+    {"row_operands", (PyCFunction)(void*)&row_operands, METH_FASTCALL, nullptr},
     {nullptr, nullptr, 0, nullptr}};
 PyModuleDef module = {PyModuleDef_HEAD_INIT, "_ltx_host", nullptr, -1, methods, nullptr, nullptr, nullptr, nullptr};
 

@@ -18,8 +18,8 @@
 
 namespace ltx {
 
-constexpr int kSkinnyMaxK = 4096;   // x chunk loop bound: K / 512 chunks per lane
-constexpr int kSkinnyMaxM = 8;
+constexpr int kSkinnyMaxK = LTX_SKINNY_MAX_K;   // x chunk loop bound: K / 512 chunks per lane
+constexpr int kSkinnyMaxM = LTX_SKINNY_MAX_ROWS;
 constexpr int kSkinnyThreads = 256;
 
 struct SkinnyArgs {

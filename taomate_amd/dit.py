@@ -38,7 +38,7 @@ import torch.nn.functional as F
 import torch.nn.modules.module as nn_module
 from torch.autograd import forward_ad
 
-from . import kernels
+from . import _native, kernels
 from .attention import CausalLTXAttention, attention_with_cache, standard_attention_forward
 from .kv_cache import LayerKVCache, _cat_cache
 
@@ -93,22 +93,12 @@ def _is_plain(m: nn.Module, cls: type) -> bool:
                      or nn_module._global_forward_hooks or nn_module._global_forward_pre_hooks))
 
 
-_autocast, _function_modes, _dispatch_modes = (torch.is_autocast_enabled, torch._C._len_torch_function_stack,
-                                               torch._C._len_torch_dispatch_stack)
-_transform, _trace = torch._C._functorch.peek_interpreter_stack, torch._C._get_tracing_state
-
-
 def _is_eager() -> bool:
     """Whether an op on plain tensors would run as it is written: no gradients,
     autocast, forward-mode level, function transform, torch function or
     dispatch mode, trace or compilation sees it."""
-    return not (torch.is_grad_enabled() or _autocast("cuda") or forward_ad._current_level >= 0
-                or _transform() is not None or _function_modes() or _dispatch_modes()
-                or _trace() is not None or torch.compiler.is_compiling())
-
-
-def _is_operand(t: torch.Tensor, x: torch.Tensor) -> bool:
-    return type(t) in (nn.Parameter, torch.Tensor) and t.dtype == x.dtype and t.is_contiguous() and t.device == x.device
+    return (not torch.compiler.is_compiling() and forward_ad._current_level < 0
+            and (_native._host or _native.host()).is_eager())
 
 
 def _row_linear(lin: nn.Module, x: torch.Tensor, act: Optional[nn.Module] = None) -> torch.Tensor:
@@ -118,11 +108,7 @@ def _row_linear(lin: nn.Module, x: torch.Tensor, act: Optional[nn.Module] = None
     if (x.is_cuda and _is_plain(lin, nn.Linear) and (act is None or _is_plain(act, nn.SiLU) and not act.inplace)
             and _is_eager()):
         w, b = lin.weight, lin.bias
-        if (type(x) is torch.Tensor and x.dtype == torch.bfloat16 and x.dim() == 2
-                and 1 <= x.shape[0] <= kernels.SKINNY_MAX_ROWS and x.shape[1] <= kernels.SKINNY_MAX_K
-                and x.shape[1] % 8 == 0 and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.data_ptr() % 16 == 0
-                and _is_operand(w, x) and w.dim() == 2 and w.shape[1] == x.shape[1] and w.data_ptr() % 16 == 0
-                and (b is None or _is_operand(b, x) and b.shape == w.shape[:1])):
+        if _native._host.row_operands(x, w, b):
             return kernels.skinny_linear(x, w, b, silu=act is not None)
     return lin(x if act is None else act(x))
 

@@ -153,9 +153,6 @@ def flash_attn(q: torch.Tensor, segments: List[KVSegment], out: torch.Tensor,
                                      segment_batch_strides)
 
 
-SKINNY_MAX_ROWS, SKINNY_MAX_K = 8, 4096
-
-
 def skinny_linear(x: torch.Tensor, weight: torch.Tensor, bias: Optional[torch.Tensor] = None,
                   silu: bool = False) -> torch.Tensor:
     """ltx_skinny_linear: act(x) @ weight.T + bias for x [M <= 8, K <= 4096]

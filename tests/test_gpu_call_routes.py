@@ -260,3 +260,17 @@ def test_timestep_mlp_keeps_what_modules_do(dev, how):
     torch.cuda.synchronize()
     assert out.dtype == want.dtype and torch.equal(out, want)
     assert calls == (2 if how == "global_hook" else 0)
+
+
+def test_timestep_mlp_takes_the_row_kernel(dev, monkeypatch):
+    """Plain modules without grad (and in inference mode): three row linears a
+    call up to 8 rows, none beyond or with gradients."""
+    m = dit.AdaLayerNormSingle(512, 6).to(dev, torch.bfloat16)
+    calls, run = [], kernels.skinny_linear
+    monkeypatch.setattr(kernels, "skinny_linear", lambda *a, **k: (calls.append(1), run(*a, **k))[1])
+    seen = []
+    for ctx, rows in ((torch.no_grad, 2), (torch.inference_mode, 8), (torch.no_grad, 9), (torch.enable_grad, 2)):
+        with ctx():
+            m(torch.rand(rows, device=dev) * 1000, torch.bfloat16)
+        seen.append(len(calls))
+    assert seen == [3, 6, 6, 6]

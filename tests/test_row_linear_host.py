@@ -94,3 +94,25 @@ def test_transforms_and_traces_run_as_modules():
         torch.vmap(fn)(torch.zeros(3))
         torch.jit.trace(fn, torch.zeros(3), check_trace=False)
     assert seen == [False, False]
+
+
+class _Tensor(torch.Tensor):
+    pass
+
+
+def test_operands_that_the_row_kernel_does_not_take():
+    """CPU, wrong types, subclasses and tensors without storage are declined, not errors."""
+    from torch._subclasses.fake_tensor import FakeTensorMode
+    from taomate_amd import _native
+    ok = _native.host().row_operands
+    x, w = torch.zeros(2, 64, dtype=torch.bfloat16), torch.zeros(8, 64, dtype=torch.bfloat16)
+    with FakeTensorMode():
+        fake = torch.empty(2, 64, dtype=torch.bfloat16, device="cuda")
+    meta = torch.empty(2, 64, dtype=torch.bfloat16, device="meta")
+    for a in (x, x.float(), x.as_subclass(_Tensor), fake, meta, x.to_sparse(), None, 3):
+        assert ok(a, w, None) is False
+    held = []
+    torch.vmap(lambda t: (held.append(t), t)[1])(x)   # a transform's tensor, past its end
+    assert ok(held[0], w, None) is False
+    with pytest.raises(TypeError):
+        ok(x, w)
