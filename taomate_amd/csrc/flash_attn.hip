@@ -2142,13 +2142,22 @@ struct Split {
 // and the keys are long: tail 96, 5 against 2 ranges, D = 128 at 41: 27.6 / 28.0,
 // 72: 36.1 / 39.9; D = 64 at 41: 20.0 / 22.4; fp8 at 24: 26.6 / 29.9, 48: 35.9 / 46.5.
 //
-// Token-major calls came from a staged kernel whose pieces filled every slot,
-// three workgroups per CU at D = 64, and keep at least as many ranges in a
-// partial round (V2A 75 x 1152: error 1.020 times with 4 instead of 8), or take
-// float32 partials where fewer are faster (tail 80 at D = 64, KT 18: 3 ranges in
-// float32 16.0 us, 8 in bf16 19.2), or run whole over few keys (tail 160 D = 128 at
-// 18: 24.4 against 28.9 us in 3 ranges in float32).  Behind whole rounds four bf16 ranges are as exact as
-// eight (1.0005), two or three are not.
+// Token-major calls came from a staged kernel whose pieces filled every slot
+// (three workgroups per CU at D = 64, where up to 768 q-tiles were one round).  In
+// a partial round they keep at least as many bf16 ranges (V2A 75 x 1152: error
+// 1.020 times with 4 instead of 8), or run whole over few keys (tail 160 at D = 128,
+// whole / 3 ranges, KT 27: 34.0 / 29.4; tail 192, whole / 2, 41: 48.6 / 46.2), or,
+// at D = 64, take float32 partials where fewer ranges are faster:
+//   tails up to 64: 8 bf16 ranges (tail 64 at KT 18: 14.4, 4 in float32 15.2)
+//   more: one piece per CU in float32, per slot over longer keys (tail 80, 3 / 5
+//     ranges, KT 41: 21.9 / 25.5, 162: 49.2 / 46.8; tail 96, 2 / 5, 41: 25.9 / 24.5,
+//     72: 35.2 / 29.3; tail 160, whole / 3, 27: 24.3 / 24.8, 41: 34.4 / 29.8), whole over
+//     few keys (tail 80, whole / 3, 11: 13.5 / 14.9, 18: 18.0 / 16.0; 128 pair units,
+//     whole / 2, 15: 22.3 / 27.5)
+//   a third to a half of the slots: the bf16 ranges of three per CU (tail 192, 4 bf16
+//     / 2 float32, KT 41: 32.5 / 34.8, 162: 83.8 / 97.1)
+// Behind whole rounds four bf16 ranges are as exact as eight (1.0005) at D = 128; two
+// or three are not, nor any at D = 64, whose rows ran whole there.
 inline Split plan_split(int64_t units, int ntiles, FlashPath path, bool pair, int64_t D) {
   const Slots s = flash_slots(D, path, pair);
   if (s.slots <= 0 || units % s.slots == 0) return {units, 1, false};
