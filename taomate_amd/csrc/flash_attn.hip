@@ -107,6 +107,10 @@ __device__ __forceinline__ float quad_sum(float x) {
   return pair_sum(__uint_as_float(r[0]) + __uint_as_float(r[1]));
 }
 
+// Which kernels can store float32 partials (FlashParams::part_f32): the launch
+// plan asks no others for them.
+constexpr bool stores_f32_partials(int D, bool pair, bool token) { return !pair || (token && D == 64); }
+
 constexpr int kBM = 128;
 constexpr int kBN = 64;
 constexpr float kLog2e = 1.4426950408889634f;
@@ -1381,7 +1385,7 @@ __device__ __forceinline__ void flash_bf16_body(const FlashParams& p) {
   static_assert((PAIR ? 8 : 4) * 32 * D <= 2 * (KBUF + VBUF), "output staging region");
   const int owave = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
   const float l_tot[2] = {quad_sum(l_run[0]), quad_sum(l_run[1])};
-  finish_rows<D, !PAIR || (VTOK && D == 64)>(p, wi, b, h, qt, wave * 32, oacc, m_run, l_tot, smem + owave * 32 * D);
+  finish_rows<D, stores_f32_partials(D, PAIR, VTOK)>(p, wi, b, h, qt, wave * 32, oacc, m_run, l_tot, smem + owave * 32 * D);
 }
 
 // The 32x32x16 body: the fp8 kernels, and bf16 key-major V where the part is
@@ -1954,7 +1958,7 @@ __device__ __forceinline__ void flash_mfma32_body(const FlashParams& p) {
   static_assert(4 * 32 * (D + 8) <= 2 * KBUF && 4 * 32 * (D + 8) <= 2 * VBUF, "output staging region");
   const int owave = PAIR ? wave : (int)(threadIdx.x >> 6);
   uint16_t* stage = (PAIR && grp == 1 ? &vbuf[0][0] : &kbuf[0][0]) + owave * 32 * (D + 8);
-  finish_tile<D, !PAIR>(p, wi, b, h, qt, owave * 32 + (int)(threadIdx.x & 31), oacc, m_run, pair_sum(l_run), stage);
+  finish_tile<D, stores_f32_partials(D, PAIR, false)>(p, wi, b, h, qt, owave * 32 + (int)(threadIdx.x & 31), oacc, m_run, pair_sum(l_run), stage);
 }
 
 // KV operands of a kernel instance: bf16 with key-major V (kKeyMajorV32: on
@@ -2157,7 +2161,8 @@ struct Split {
 //   a third to a half of the slots: the bf16 ranges of three per CU (tail 192, 4 bf16
 //     / 2 float32, KT 41: 32.5 / 34.8, 162: 83.8 / 97.1)
 // Behind whole rounds four bf16 ranges are as exact as eight (1.0005) at D = 128; two
-// or three are not, nor any at D = 64, whose rows ran whole there.
+// or three are not, nor any at D = 64, whose rows ran whole there.  (The pair units'
+// ranges at D = 128 are the ones that the staged kernel had.)
 inline Split plan_split(int64_t units, int ntiles, FlashPath path, bool pair, int64_t D) {
   const Slots s = flash_slots(D, path, pair);
   if (s.slots <= 0 || units % s.slots == 0) return {units, 1, false};
@@ -2178,7 +2183,7 @@ inline Split plan_split(int64_t units, int ntiles, FlashPath path, bool pair, in
     if (two_per_cu && 2 * tail > s.cus && ntiles < (d64 || 3 * tail > S ? 36 : 24)) n = 1;
     if (f32 && ntiles < (2 * tail < s.cus || two_per_cu ? 16 : 27)) n = 1;
   } else if (token) {
-    f32 = d64 || n < 4;
+    f32 = d64 || (two_per_cu && n < 4);
   } else if (two_per_cu && one_round && n >= 2 && n <= (fp8 ? 4 : 3) && ntiles >= (fp8 ? 36 : d64 ? 40 : 72)) {
     n = S / tail;
   }
@@ -2443,6 +2448,8 @@ static int flash_attn_fwd_impl(const void* q, int64_t B, int64_t Lq, int64_t H, 
     if (workspace != nullptr) {
       sp = plan_split(nu, p.tile_start[n], path, p.pair != 0, D);
       if (sp.bytes(nu, per_unit, D) > workspace_bytes) sp = {nu, 1, false};
+      LTX_REQUIRE(!sp.f32 || stores_f32_partials((int)D, p.pair != 0, path == kPathTokenMajor),
+                  "ltx_flash_attn_fwd: a launch plan with float32 partials that its kernel does not store");
     }
     p.n_full = (int)sp.n_full;
     p.split = sp.n;

@@ -119,23 +119,14 @@ def _whole(q, seg, out, frame):
                  torch.cuda.current_stream().cuda_stream)
 
 
-@pytest.mark.parametrize("layout,B,Lq,H,D,keys", [
-    ("key", 1, 620, 32, 128, 4000), ("key", 2, 300, 32, 64, 5000), ("key", 2, 620, 32, 64, 5000),
-    ("key", 1, 1370, 32, 128, 7000), ("token", 2, 620, 32, 128, 4000), ("token", 1, 300, 32, 64, 2600),
-    ("token", 2, 512, 32, 64, 2000), ("token", 2, 1152, 32, 64, 1152), ("token", 1, 2423, 32, 128, 1152),
-    ("fp8", 1, 620, 32, 64, 1650), ("fp8", 2, 300, 32, 128, 2640), ("fp8", 2, 620, 32, 128, 3300),
-    ("fp8", 1, 1370, 32, 64, 4950)])
-def test_split_keeps_float32_sums(dev, layout, B, Lq, H, D, keys):
-    """Tails that are split with float32 partials, one case per branch of the
-    launch plan: the error against float64 is the whole q-tiles' (bf16
-    partials of all rows make it 1.22 times that).  Both share P's rounding
-    and the output's; over the 1e5 and more values compared, what is left
-    differs by well under 1 %."""
+def _split_case(dev, layout, B, Lq, H, D, keys, frame=330):
+    """A call with its launch plan and with whole q-tiles: both outputs, their
+    root mean square errors against float64 on a few heads."""
     g = torch.Generator(device=dev)
     g.manual_seed(keys + Lq)
     r = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
     q, k, v = r(B, Lq, H, D), r(B, keys, H, D), r(B, keys, H, D)
-    frame = 330 if layout == "fp8" else 0
+    frame = frame if layout == "fp8" else 0
     if layout == "fp8":
         seg, k, v = _fp8_cache(k, v, frame, dev)
     elif layout == "key":
@@ -148,14 +139,69 @@ def test_split_keeps_float32_sums(dev, layout, B, Lq, H, D, keys):
     kernels.flash_attn(q, [seg], out, frame_tokens=frame)
     _whole(q, seg, whole, frame)
     torch.cuda.synchronize()
-    assert not torch.equal(out, whole)   # the plan does split
     err = [0.0, 0.0]
     for b, h in ((0, 0), (B - 1, H - 1), (0, H // 2), (B - 1, 5)):
         p = ((q[b, :, h].double() @ k[b, :, h].double().t().contiguous()) / math.sqrt(D)).softmax(-1)
         ref = p @ v[b, :, h].double()
         for i, o in enumerate((out, whole)):
             err[i] += (o[b, :, h].double() - ref).square().sum().item()
-    assert math.sqrt(err[0] / err[1]) <= 1.02
+    return out, whole, math.sqrt(err[0]), math.sqrt(err[1])
+
+
+@pytest.mark.parametrize("keys", [640, 2560, 5120])
+@pytest.mark.parametrize("B,H,qtiles", [(2, 32, 1), (1, 32, 3), (2, 32, 3), (1, 32, 7), (2, 32, 9), (2, 32, 11),   # 4-wave
+                                        (1, 32, 2), (2, 32, 4), (2, 32, 10), (2, 32, 12), (2, 24, 14)])          # pair units
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("layout,frame", [("key", 0), ("token", 0), ("fp8", 320), ("fp8", 160)])
+def test_launch_plan_against_whole_tiles(dev, layout, frame, D, B, H, qtiles, keys):
+    """Every kernel (fp8 in frames of whole 64-key tiles and not) with tails of a partial round and behind whole rounds, over
+    few and many keys: bf16 partials add one rounding of the output's size to
+    the two of P and the output (sqrt(3 / 2) = 1.22 times the error), float32
+    partials none."""
+    _, _, err, whole = _split_case(dev, layout, B, qtiles * 128 - 20, H, D, keys, frame)
+    assert err <= 1.3 * whole
+
+
+@pytest.mark.parametrize("layout,B,Lq,H,D,keys", [
+    ("key", 1, 620, 32, 128, 4000), ("key", 2, 300, 32, 64, 5000), ("key", 2, 620, 32, 64, 5000),
+    ("key", 1, 1370, 32, 128, 7000), ("token", 2, 620, 32, 128, 4000), ("token", 1, 300, 32, 64, 2600),
+    ("token", 2, 512, 32, 64, 2000), ("token", 2, 1152, 32, 64, 1152), ("token", 1, 2423, 32, 128, 1152),
+    ("fp8", 1, 620, 32, 64, 1650), ("fp8", 2, 300, 32, 128, 2640), ("fp8", 2, 620, 32, 128, 3300),
+    ("fp8", 1, 1370, 32, 64, 4950)])
+def test_split_keeps_float32_sums(dev, layout, B, Lq, H, D, keys):
+    """Tails that are split with float32 partials, one case per branch of the
+    launch plan: the error against float64 is the whole q-tiles' (bf16
+    partials of all rows make it 1.22 times that).  Both share P's rounding
+    and the output's; over the 1e5 and more values compared, what is left
+    differs by well under 1 %."""
+    out, whole, err, err_whole = _split_case(dev, layout, B, Lq, H, D, keys)
+    assert not torch.equal(out, whole)   # the plan does split
+    assert err <= 1.02 * err_whole
+
+
+@pytest.mark.parametrize("counts", [(5000, 37), (0, 5000), (1300, 2501)])
+def test_key_counts_over_float32_ranges(dev, counts):
+    """Per-row key counts where the plan cuts the keys into ranges with float32
+    partials: ranges past a row's count hold nothing."""
+    B, Lq, H, D, n = 2, 300, 32, 64, 5000
+    g = torch.Generator(device=dev)
+    g.manual_seed(sum(counts))
+    r = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+    q, k, v = r(B, Lq, H, D), r(B, n, H, D), r(B, n, H, D)
+    store = v.permute(0, 2, 3, 1).contiguous()
+    out = torch.empty_like(q)
+    lse = torch.empty(B, H, Lq, dtype=torch.float32, device=dev)
+    kernels.flash_attn(q, [KVSegment(k, store.permute(0, 3, 1, 2))], out, lse=lse, key_lens=list(counts))
+    torch.cuda.synchronize()
+    for b, m in enumerate(counts):
+        for h in (0, H - 1):
+            if m == 0:
+                assert (out[b, :, h] == 0).all() and (lse[b, h] == float("-inf")).all()
+                continue
+            s = q[b, :, h].double() @ k[b, :m, h].double().t().contiguous() / math.sqrt(D)
+            ref = s.softmax(-1) @ v[b, :m, h].double()
+            assert (out[b, :, h].double() - ref).abs().max().item() <= _bound(v)
+            assert (lse[b, h].double() - s.logsumexp(-1)).abs().max().item() <= 2.0 ** -9
 
 
 @pytest.mark.parametrize("B,L,H,D", [(2, 1, 8, 64), (1, 33, 32, 128), (2, 75, 32, 64)])
