@@ -2143,8 +2143,11 @@ struct Split {
 //   above: no split gains (tail 416 and 448: 1.03 to 1.3 times as long up to 6912 keys)
 // More ranges in bf16 than the base cost no exactness: grids of one partial
 // round take one piece per slot where the base gives 2 or 3 ranges (fp8: 4 too)
-// and the keys are long: tail 96, 5 against 2 ranges, D = 128 at 41: 27.6 / 28.0,
-// 72: 36.1 / 39.9; D = 64 at 41: 20.0 / 22.4; fp8 at 24: 26.6 / 29.9, 48: 35.9 / 46.5.
+// and the keys are long.  Base / one per slot: tail 96 (2 / 5 ranges) D = 128 at KT
+// 41: 28.3 / 27.8, 54: 33.0 / 30.7; D = 64 at 21: 16.4 / 16.3, 31: 19.5 / 17.7; fp8 at 24: 29.9 /
+// 26.5, 48: 46.5 / 35.9; tail 112 (2 / 4) D = 128 at 41: 29.5 / 30.2, 54: 33.9 / 33.7; tail 72
+// (3 / 7) D = 128 at 41: 23.7 / 24.6, 63: 29.7 / 29.2; D = 64 at 31: 16.7 / 17.3, 41: 18.8 /
+// 18.1; fp8 at 24: 24.8 / 25.0, 36: 30.4 / 28.4.
 //
 // Token-major calls came from a staged kernel whose pieces filled every slot
 // (three workgroups per CU at D = 64, where up to 768 q-tiles were one round).  In
@@ -2184,8 +2187,8 @@ inline Split plan_split(int64_t units, int ntiles, FlashPath path, bool pair, in
     if (f32 && ntiles < (2 * tail < s.cus || two_per_cu ? 16 : 27)) n = 1;
   } else if (token) {
     f32 = d64 || (two_per_cu && n < 4);
-  } else if (two_per_cu && one_round && n >= 2 && n <= (fp8 ? 4 : 3) && ntiles >= (fp8 ? 36 : d64 ? 40 : 72)) {
-    n = S / tail;
+  } else if (two_per_cu && one_round && n >= 2 && n <= (fp8 ? 4 : 3)) {
+    if (ntiles >= (n == 2 ? (fp8 ? 24 : d64 ? 32 : 54) : (fp8 ? 36 : d64 ? 40 : 72))) n = S / tail;
   }
   if (two_per_cu && n < 2) {
     f32 = true;
